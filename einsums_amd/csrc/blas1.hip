@@ -373,18 +373,55 @@ int dot_noalloc_f64(int64_t n, double alpha, double const *x, int64_t incx, doub
 }
 
 // -------------------------------------------------------------------- ger
-template <typename T>
+// A(i,j) = beta*A(i,j) + alpha*x(i)*y(j) over rows of stride rs and columns of stride lda.
+// HBM-bound: A is written once, and read once unless beta == 0. A workgroup is 2^tr threads
+// along the rows times 256 / 2^tr along the columns; a thread owns VEC consecutive rows (one
+// 16-byte access) of GER_COLS columns, whose reads are issued together. The row width follows
+// m, so that a short m leaves no lane idle: the rank-0 times tensor product of a gradient is
+// a 1 x N outer product, which a fixed 64-row block ran with one lane in 64 (16.8M doubles
+// 1706 us plus 21 us to zero them first; in this form, with the factor on A fused, 46 us = 5.8 TB/s).
+constexpr int GER_COLS = 4;
+
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void ger_kernel(int64_t m, int64_t n, T alpha, T const *__restrict__ x, int64_t incx,
-                                                  T const *__restrict__ y, int64_t incy, T *__restrict__ A, int64_t lda) {
-    int64_t const i = int64_t(blockIdx.x) * 64 + (threadIdx.x & 63);
-    if (i >= m) return;
-    T const xi = alpha * x[i * incx];
-    for (int64_t j = int64_t(blockIdx.y) * 4 + (threadIdx.x >> 6); j < n; j += int64_t(gridDim.y) * 4)
-        A[i + j * lda] += xi * y[j * incy];
+                                                  T const *__restrict__ y, int64_t incy, T beta, T *__restrict__ A,
+                                                  int64_t rs, int64_t lda, int tr) {
+    struct alignas(VEC * sizeof(T)) Vec {
+        T v[VEC];
+    };
+    int const lc    = int(threadIdx.x) >> tr;
+    int const cols  = 256 >> tr;
+    int64_t const i = ((int64_t(blockIdx.x) << tr) + (threadIdx.x & ((1u << tr) - 1))) * VEC;
+    if (i >= m) return; // VEC divides m
+    T xi[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) xi[v] = alpha * x[(i + v) * incx];
+    int64_t const step = int64_t(cols) * GER_COLS;
+    for (int64_t j0 = int64_t(blockIdx.y) * step + lc; j0 < n; j0 += int64_t(gridDim.y) * step) {
+        Vec c[GER_COLS];
+        T yj[GER_COLS];
+#pragma unroll
+        for (int u = 0; u < GER_COLS; ++u) {
+            int64_t const j = j0 + u * cols;
+            yj[u]           = j < n ? y[j * incy] : T(0);
+            if (beta != T(0) && j < n) c[u] = *reinterpret_cast<Vec const *>(A + i * rs + j * lda);
+        }
+#pragma unroll
+        for (int u = 0; u < GER_COLS; ++u) {
+            int64_t const j = j0 + u * cols;
+            if (j >= n) break;
+#pragma unroll
+            for (int v = 0; v < VEC; ++v)
+                c[u].v[v] = beta != T(0) ? fma(xi[v], yj[u], beta * c[u].v[v]) : xi[v] * yj[u];
+            *reinterpret_cast<Vec *>(A + i * rs + j * lda) = c[u];
+        }
+    }
 }
 
+// ger with a factor on A (the reference's ger is the beta == 1 case). alpha == 0 leaves A
+// alone, as in BLAS; a caller with beta != 1 scales A itself then.
 template <typename T>
-int ger_impl(int64_t m, int64_t n, T alpha, T const *x, int64_t incx, T const *y, int64_t incy, T *A, int64_t lda,
+int ger_impl(int64_t m, int64_t n, T alpha, T const *x, int64_t incx, T const *y, int64_t incy, T beta, T *A, int64_t lda,
              hipStream_t stream) {
     if (m < 0) return fail(-1, "ger: m < 0");
     if (n < 0) return fail(-2, "ger: n < 0");
@@ -394,10 +431,27 @@ int ger_impl(int64_t m, int64_t n, T alpha, T const *x, int64_t incx, T const *y
     if (m == 0 || n == 0 || alpha == T(0)) return EIN_SUCCESS;
     if (incx < 0) x = x - (m - 1) * incx;
     if (incy < 0) y = y - (n - 1) * incy;
-    int64_t rb = ceil_div(m, 64);
-    int64_t cb = std::min<int64_t>(ceil_div(n, 4), std::max<int64_t>(1, int64_t(num_cus()) * 8 / rb));
-    cb         = std::min<int64_t>(cb, 65535);
-    ger_kernel<T><<<dim3(uint32_t(rb), uint32_t(cb)), 256, 0, stream>>>(m, n, alpha, x, incx, y, incy, A, lda);
+    int64_t rs = 1;
+    if (m == 1 && n > 1) { // one row: its elements become the rows, lda apart
+        std::swap(m, n);
+        std::swap(x, y);
+        std::swap(incx, incy);
+        rs  = lda;
+        lda = 1;
+    }
+    constexpr int VW = 16 / int(sizeof(T));
+    bool const vec   = rs == 1 && m % VW == 0 && (n == 1 || lda % VW == 0) && reinterpret_cast<uintptr_t>(A) % 16 == 0;
+    int64_t const r  = vec ? m / VW : m; // threads along the rows
+    int tr           = 0;
+    while (tr < 8 && (int64_t{1} << tr) < r) ++tr;
+    int64_t const rb = ceil_div(r, int64_t{1} << tr);
+    int64_t const cb = std::min<int64_t>(ceil_div(n, int64_t(256 >> tr) * GER_COLS), 65535);
+    if (rb > 0x7fffffff) return fail(EIN_ERROR_UNSUPPORTED, "ger: more than 2^39 rows");
+    dim3 const grid{uint32_t(rb), uint32_t(cb)};
+    if (vec)
+        ger_kernel<T, VW><<<grid, 256, 0, stream>>>(m, n, alpha, x, incx, y, incy, beta, A, rs, lda, tr);
+    else
+        ger_kernel<T, 1><<<grid, 256, 0, stream>>>(m, n, alpha, x, incx, y, incy, beta, A, rs, lda, tr);
     EIN_LAUNCH_CHECK();
     return EIN_SUCCESS;
 }
@@ -532,10 +586,10 @@ template int gemv_impl<float>(char, int64_t, int64_t, float, float const *, int6
 template int dot_impl<double>(int64_t, double, double const *, int64_t, double const *, int64_t, double, double *,
                               hipStream_t);
 template int dot_impl<float>(int64_t, float, float const *, int64_t, float const *, int64_t, float, float *, hipStream_t);
-template int ger_impl<double>(int64_t, int64_t, double, double const *, int64_t, double const *, int64_t, double *,
+template int ger_impl<double>(int64_t, int64_t, double, double const *, int64_t, double const *, int64_t, double, double *,
                               int64_t, hipStream_t);
-template int ger_impl<float>(int64_t, int64_t, float, float const *, int64_t, float const *, int64_t, float *, int64_t,
-                             hipStream_t);
+template int ger_impl<float>(int64_t, int64_t, float, float const *, int64_t, float const *, int64_t, float, float *,
+                             int64_t, hipStream_t);
 template int dirprod_impl<double>(int64_t, double, double const *, int64_t, double const *, int64_t, double, double *,
                                   int64_t, hipStream_t);
 template int dirprod_impl<float>(int64_t, float, float const *, int64_t, float const *, int64_t, float, float *, int64_t,
@@ -573,11 +627,11 @@ int ein_dot_f64_noalloc(int64_t n, double alpha, const double *x, int64_t incx, 
 }
 int ein_ger_f64(int64_t m, int64_t n, double alpha, const double *x, int64_t incx, const double *y, int64_t incy, double *A,
                 int64_t lda, ein_stream_t stream) {
-    return ein::ger_impl<double>(m, n, alpha, x, incx, y, incy, A, lda, ein::as_stream(stream));
+    return ein::ger_impl<double>(m, n, alpha, x, incx, y, incy, 1.0, A, lda, ein::as_stream(stream));
 }
 int ein_ger_f32(int64_t m, int64_t n, float alpha, const float *x, int64_t incx, const float *y, int64_t incy, float *A,
                 int64_t lda, ein_stream_t stream) {
-    return ein::ger_impl<float>(m, n, alpha, x, incx, y, incy, A, lda, ein::as_stream(stream));
+    return ein::ger_impl<float>(m, n, alpha, x, incx, y, incy, 1.0f, A, lda, ein::as_stream(stream));
 }
 int ein_dirprod_f64(int64_t n, double alpha, const double *x, int64_t incx, const double *y, int64_t incy, double beta,
                     double *z, int64_t incz, ein_stream_t stream) {

@@ -278,9 +278,9 @@ int einsum_execute(int alg, T cp, ein_tensor_desc const &C, T *c, T abp, ein_ten
         bool const row = scj == 1 && sci >= std::max<int64_t>(1, ej);
         if (!col && !row) break;
         if (used) *used = EIN_ALG_GER;
-        EIN_TRY(tensor_scale<T>(C, c, cp, stream));
-        if (col) return ger_impl<T>(ei, ej, abp, a, sx, b, sy, c, std::max<int64_t>(1, scj), stream);
-        return ger_impl<T>(ej, ei, abp, b, sy, a, sx, c, std::max<int64_t>(1, sci), stream);
+        if (abp == T(0)) return tensor_scale<T>(C, c, cp, stream);
+        if (col) return ger_impl<T>(ei, ej, abp, a, sx, b, sy, cp, c, std::max<int64_t>(1, scj), stream);
+        return ger_impl<T>(ej, ei, abp, b, sy, a, sx, cp, c, std::max<int64_t>(1, sci), stream);
     }
     case EIN_ALG_GEMV: {
         // matrix operand M (labels: targets + links), vector operand V (links only)
