@@ -12,12 +12,14 @@
 // and K(a,c) with D(b,d), so both can be accumulated from one read of g: half the HBM traffic
 // of the two calls, which is what bounds them (0.25 flop per byte).
 //
-// Kernel 1: workgroup (a, one or four b's) reads the slabs g(a,b,:,:) of its b's. Wave w
-// takes the rows c = w, w+W, ... (W = 4 or 16 waves); its lanes run over d. Per lane it keeps
+// For n <= 64, kernel 1: workgroup (a, four b's) reads the slabs g(a,b,:,:) of its b's. Wave w
+// takes the rows c = w, w+4, ...; its lanes run over d. Per lane it keeps
 // K partials per row; J(a,b) is complete inside the workgroup and is written directly, K is
 // written as one partial row per chunk. Kernel 2 adds the chunks' K partials in chunk order
-// and forms F (deterministic: fixed summation trees, no atomics). n <= 128. For even n <= 64
-// with 16-byte aligned rows, kernel 1 reads two elements per lane (fock_jk16_kernel).
+// and forms F (deterministic: fixed summation trees, no atomics). For even n with 16-byte
+// aligned rows, kernel 1 reads two elements per lane (fock_jk16_kernel). For 64 < n <= 128 a
+// slab is large enough to fill a CU's loads, and one workgroup per CU streams its share of all
+// slabs (fock_jk_stream_kernel). n <= 128.
 #include <algorithm>
 #include <string>
 
@@ -29,15 +31,14 @@ namespace {
 
 constexpr int FOCK_MAX_N = 128;
 
-// NPL = elements of a row per lane (1 for n <= 64, 2 for n <= 128); WAVES = 4 or 16;
-// MR >= ceil(n / WAVES) rows c per wave; BC = b's per workgroup. Each lane keeps the
+// n <= 64. MR >= ceil(n / 4) rows c per wave; BC = b's per workgroup. Each lane keeps the
 // D(c, d) of its own (c, d) positions in registers (the same for every slab), so no LDS
 // staging or barrier precedes the slab loads: all of a workgroup's slab reads are in
 // flight at once, and the many resident workgroups keep HBM busy.
-template <int NPL, int WAVES, int MR, int BC>
-__global__ __launch_bounds__(64 * WAVES) void fock_jk_kernel(int n, double const *__restrict__ g,
-                                                             double const *__restrict__ D, int64_t ldd,
-                                                             double *__restrict__ J, double *__restrict__ Kp) {
+template <int MR, int BC>
+__global__ __launch_bounds__(256) void fock_jk_kernel(int n, double const *__restrict__ g, double const *__restrict__ D,
+                                                      int64_t ldd, double *__restrict__ J, double *__restrict__ Kp) {
+    constexpr int WAVES = 4, NPL = 1;
     __shared__ double red[WAVES][BC];
     int const a    = int(blockIdx.x);
     int const ch   = int(blockIdx.y);
@@ -184,6 +185,153 @@ __global__ __launch_bounds__(256) void fock_jk16_kernel(int n, double const *__r
     }
 }
 
+// 64 < n <= 128: one workgroup of 16 waves per CU takes `units` consecutive slabs
+// s = a*n + b, and holds the next slab's loads in registers while it works on one. HBM-bound:
+// one slab (34 to 131 KB) in flight per CU covers the latency, and no workgroup start, D read
+// or K reduction comes between two slabs of the same a. MR = ceil(n / 16) rows c = wave + 16 i;
+// VEC: a lane reads d = 2l, 2l+1 as 16 bytes (even n, 16-byte aligned rows), otherwise d = l
+// and l + 64. All loads are unconditional, from clamped addresses, so that the wait before a
+// slab counts exactly the loads behind it; what lies outside is dropped where it is summed.
+// J(a,b) sums its waves from LDS at the end; K is written per a as piece 2w (the first a of
+// workgroup w) or 2w+1. One workgroup per slab, whose shuffle reductions and start nothing
+// overlapped, took 195 + 13.5 us at n = 96 (3.4 TB/s over the call). Now, per call: n = 65 47 us
+// (before 77), 96 126 us = 5.4 TB/s (202), 97 161 (314), 112 215 (435), 127 425 (620), 128 362 (621).
+constexpr int FOCK_WAVES = 16, FOCK_UNITS = 64; // LDS for the J sums of 64 slabs
+
+template <int MR, bool VEC>
+__global__ __launch_bounds__(64 * FOCK_WAVES) void fock_jk_stream_kernel(int n, int units, double const *__restrict__ g,
+                                                                         double const *__restrict__ D, int64_t ldd,
+                                                                         double *__restrict__ J,
+                                                                         double *__restrict__ Kp) {
+    // D(c,d) in registers, or in LDS where two slabs of x leave no room for it in the 128 of a
+    // 1024-thread workgroup (n = 127 then spilled: 672 us)
+    constexpr bool D_LDS = !VEC || MR == 8;
+    __shared__ double jred[FOCK_UNITS][FOCK_WAVES];
+    __shared__ double dl[D_LDS ? FOCK_MAX_N * FOCK_MAX_N : 1];
+    int const wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    int const lane = int(threadIdx.x) & 63;
+    int const nn   = n * n;
+    if constexpr (D_LDS) {
+        for (int c = wave; c < n; c += FOCK_WAVES)
+            for (int d = lane; d < n; d += 64) dl[c * n + d] = D[int64_t(c) * ldd + d];
+        __syncthreads();
+    }
+    int const s0 = int(blockIdx.x) * units, s1 = s0 + units < nn ? s0 + units : nn;
+    bool const in0 = !VEC || 2 * lane < n, in1 = VEC || lane + 64 < n; // the lane's two elements
+    bool const last_in = wave + FOCK_WAVES * (MR - 1) < n;             // its last row
+    int const d0 = VEC ? (in0 ? 2 * lane : n - 2) : lane;
+    int const d1 = VEC ? d0 + 1 : (in1 ? lane + 64 : n - 1);
+    auto load_row = [&](double const *__restrict__ row, double (&v)[2]) {
+        if constexpr (VEC) {
+            double2 const t = *reinterpret_cast<double2 const *>(row + d0);
+            v[0] = t.x;
+            v[1] = t.y;
+        } else {
+            v[0] = row[d0];
+            v[1] = row[d1];
+        }
+    };
+    int row[MR]; // offset of the wave's rows in a slab
+    double dc[D_LDS ? 1 : MR][2];
+#pragma unroll
+    for (int i = 0; i < MR; ++i) {
+        int const c = i < MR - 1 || last_in ? wave + FOCK_WAVES * i : n - 1;
+        row[i]      = c * n;
+        if constexpr (!D_LDS) load_row(D + int64_t(c) * ldd, dc[i]);
+    }
+    auto load = [&](int s, int b, double (&x)[MR][2], double (&db)[2]) {
+        double const *__restrict__ slab = g + int64_t(s) * nn;
+        load_row(D + int64_t(b) * ldd, db);
+#pragma unroll
+        for (int i = 0; i < MR; ++i) load_row(slab + row[i], x[i]);
+    };
+    double kacc[MR];
+#pragma unroll
+    for (int i = 0; i < MR; ++i) kacc[i] = 0.0;
+    int const a0 = s0 / n;
+    int a = a0, b = s0 - a0 * n;
+    auto write_k = [&]() {
+        double *__restrict__ kp = Kp + int64_t(2 * int(blockIdx.x) + (a != a0 ? 1 : 0)) * n;
+#pragma unroll
+        for (int i = 0; i < MR; ++i) {
+            double const s = wave_reduce_sum(in0 ? kacc[i] : 0.0);
+            if (lane == 0 && (i < MR - 1 || last_in)) kp[wave + FOCK_WAVES * i] = s;
+            kacc[i] = 0.0;
+        }
+    };
+    auto work = [&](int s, double (&x)[MR][2], double (&db)[2]) {
+        double jsum = 0.0;
+        int e0 = d0, e1 = d1;
+        if constexpr (D_LDS) asm volatile("" : "+v"(e0), "+v"(e1)); // read each time, not kept in registers
+#pragma unroll
+        for (int i = 0; i < MR; ++i) {
+            double const y = in1 ? x[i][1] : 0.0;
+            double const j = x[i][0] * (D_LDS ? dl[row[i] + e0] : dc[D_LDS ? 0 : i][0]) +
+                             y * (D_LDS ? dl[row[i] + e1] : dc[D_LDS ? 0 : i][1]);
+            jsum += i < MR - 1 || last_in ? j : 0.0;
+            kacc[i] += x[i][0] * db[0] + y * db[1];
+        }
+        jsum = wave_reduce_sum(in0 ? jsum : 0.0);
+        if (lane == 0) jred[s - s0][wave] = jsum;
+        if (++b == n) {
+            write_k();
+            b = 0;
+            ++a;
+        }
+    };
+    double xa[MR][2], xb[MR][2], dba[2], dbb[2];
+    auto next_b = [&](int ahead) { return b + ahead < n ? b + ahead : b + ahead - n; };
+    load(s0, b, xa, dba);
+    int s = s0;
+    for (; s + 2 < s1; s += 2) {
+        load(s + 1, next_b(1), xb, dbb);
+        work(s, xa, dba);
+        load(s + 2, next_b(1), xa, dba); // b has moved on
+        work(s + 1, xb, dbb);
+    }
+    if (s + 1 < s1) {
+        load(s + 1, next_b(1), xb, dbb);
+        work(s, xa, dba);
+        work(s + 1, xb, dbb);
+    } else {
+        work(s, xa, dba);
+    }
+    if (b != 0) write_k();
+    __syncthreads();
+    if (int(threadIdx.x) < s1 - s0) {
+        double j = 0.0;
+#pragma unroll
+        for (int w = 0; w < FOCK_WAVES; ++w) j += jred[threadIdx.x][w];
+        J[s0 + int(threadIdx.x)] = j;
+    }
+}
+
+// F(a,c) from J and the K pieces of row a, in workgroup order.
+__global__ __launch_bounds__(256) void fock_finish_pieces_kernel(int n, int units, double const *__restrict__ J,
+                                                                 double const *__restrict__ Kp, double alpha_j,
+                                                                 double alpha_k, double beta, double *__restrict__ F,
+                                                                 int64_t ldf) {
+    int const e = int(blockIdx.x) * 256 + int(threadIdx.x);
+    if (e >= n * n) return;
+    int const a = e / n, c = e - a * n;
+    double k = 0.0;
+    for (int w = a * n / units; w <= (a * n + n - 1) / units; ++w)
+        k += Kp[int64_t(2 * w + (w * units / n != a ? 1 : 0)) * n + c];
+    double *fp = F + int64_t(a) * ldf + c;
+    double v   = alpha_j * J[e] + alpha_k * k;
+    if (beta != 0.0) v += beta * *fp;
+    *fp = v;
+}
+
+template <int MR>
+void launch_stream(bool vec, int grid, int n, int units, double const *g, double const *D, int64_t ldd, double *J,
+                   double *Kp, hipStream_t stream) {
+    if (vec)
+        fock_jk_stream_kernel<MR, true><<<grid, 64 * FOCK_WAVES, 0, stream>>>(n, units, g, D, ldd, J, Kp);
+    else
+        fock_jk_stream_kernel<MR, false><<<grid, 64 * FOCK_WAVES, 0, stream>>>(n, units, g, D, ldd, J, Kp);
+}
+
 // F(a,c) = beta*F(a,c) + alpha_j*J(a,c) + alpha_k*sum_chunk Kp(a,chunk,c), chunks in order.
 __global__ __launch_bounds__(256) void fock_finish_kernel(int n, int chunks, double const *__restrict__ J,
                                                           double const *__restrict__ Kp, double alpha_j, double alpha_k,
@@ -218,7 +366,30 @@ int fock_jk_f64(int64_t n, double const *g, double const *D, int64_t ldd, double
                                                " (use the two einsum calls)");
     if (n == 0) return EIN_SUCCESS;
     if (g == nullptr || D == nullptr || F == nullptr) return fail(-2, "fock_jk: null pointer");
-    int const bc     = n <= 64 ? 4 : 1; // the kernels' BC
+    bool const wide = n % 2 == 0 && ldd % 2 == 0 && reinterpret_cast<uintptr_t>(g) % 16 == 0 &&
+                      reinterpret_cast<uintptr_t>(D) % 16 == 0;
+    int const ni    = int(n);
+    if (n > 64) {
+        // units <= FOCK_UNITS <= n - 1, so a workgroup's slabs meet at most two values of a
+        int const units = int(std::min<int64_t>(ceil_div(n * n, num_cus()), FOCK_UNITS));
+        int const grid  = int(ceil_div(n * n, units));
+        void *ws        = nullptr;
+        EIN_TRY(workspace(stream, (size_t(n) * size_t(n) + 2 * size_t(grid) * size_t(n)) * sizeof(double), &ws));
+        double *J  = static_cast<double *>(ws);
+        double *Kp = J + size_t(n) * size_t(n);
+        switch (int(ceil_div(n, FOCK_WAVES))) {
+        case 5: launch_stream<5>(wide, grid, ni, units, g, D, ldd, J, Kp, stream); break;
+        case 6: launch_stream<6>(wide, grid, ni, units, g, D, ldd, J, Kp, stream); break;
+        case 7: launch_stream<7>(wide, grid, ni, units, g, D, ldd, J, Kp, stream); break;
+        default: launch_stream<8>(wide, grid, ni, units, g, D, ldd, J, Kp, stream); break;
+        }
+        EIN_LAUNCH_CHECK();
+        fock_finish_pieces_kernel<<<uint32_t(ceil_div(n * n, 256)), 256, 0, stream>>>(ni, units, J, Kp, alpha_j, alpha_k,
+                                                                                    beta, F, ldf);
+        EIN_LAUNCH_CHECK();
+        return EIN_SUCCESS;
+    }
+    constexpr int bc = 4; // the kernels' BC
     int const chunks = int(ceil_div(n, bc));
     void *ws = nullptr;
     size_t const j_bytes = size_t(n) * size_t(n) * sizeof(double);
@@ -227,11 +398,6 @@ int fock_jk_f64(int64_t n, double const *g, double const *D, int64_t ldd, double
     double *J  = static_cast<double *>(ws);
     double *Kp = J + size_t(n) * size_t(n);
     dim3 grid{uint32_t(n), uint32_t(chunks)};
-    int const ni = int(n);
-    // two elements per lane for even n <= 64 (a one-row-per-load form for 64 < n <= 128
-    // measured slower than the kernel below it: 215 against 201 us cold at n = 96)
-    bool const wide = n % 2 == 0 && n <= 64 && ldd % 2 == 0 && reinterpret_cast<uintptr_t>(g) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(D) % 16 == 0;
     if (wide && n <= 32)
         fock_jk16_kernel<4, 4><<<grid, 256, 0, stream>>>(ni, g, D, ldd, J, Kp);
     else if (wide && n <= 48)
@@ -239,15 +405,11 @@ int fock_jk_f64(int64_t n, double const *g, double const *D, int64_t ldd, double
     else if (wide)
         fock_jk16_kernel<8, 4><<<grid, 256, 0, stream>>>(ni, g, D, ldd, J, Kp);
     else if (n <= 32)
-        fock_jk_kernel<1, 4, 8, 4><<<grid, 256, 0, stream>>>(ni, g, D, ldd, J, Kp);
+        fock_jk_kernel<8, 4><<<grid, 256, 0, stream>>>(ni, g, D, ldd, J, Kp);
     else if (n <= 48)
-        fock_jk_kernel<1, 4, 12, 4><<<grid, 256, 0, stream>>>(ni, g, D, ldd, J, Kp);
-    else if (n <= 64)
-        fock_jk_kernel<1, 4, 16, 4><<<grid, 256, 0, stream>>>(ni, g, D, ldd, J, Kp);
-    else if (n <= 96)
-        fock_jk_kernel<2, 16, 6, 1><<<grid, 1024, 0, stream>>>(ni, g, D, ldd, J, Kp);
+        fock_jk_kernel<12, 4><<<grid, 256, 0, stream>>>(ni, g, D, ldd, J, Kp);
     else
-        fock_jk_kernel<2, 16, 8, 1><<<grid, 1024, 0, stream>>>(ni, g, D, ldd, J, Kp);
+        fock_jk_kernel<16, 4><<<grid, 256, 0, stream>>>(ni, g, D, ldd, J, Kp);
     EIN_LAUNCH_CHECK();
     fock_finish_kernel<<<uint32_t(ceil_div(n * n, 256)), 256, 0, stream>>>(int(n), chunks, J, Kp, alpha_j, alpha_k, beta,
                                                                          F, ldf);
