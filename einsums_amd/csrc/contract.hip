@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "contract.hpp"
@@ -1074,47 +1075,211 @@ int ein_contract_f32(float c_prefactor, const ein_tensor_desc *C, float *c, floa
 // ===================================================== grouped launches
 //
 // A grouped plan holds many independent contractions (the blocks of a block-sparse
-// einsum, a batch of uneven GEMMs). Each becomes a gather-GEMM problem; all their tiles
-// form one list sorted by contraction length (longest first) and a persistent launch of
-// about two workgroups per CU walks the list with a fixed stride -- one launch per wave
-// of items whose outputs do not overlap. Descriptors live in device memory, so executing
-// a plan is a pure kernel launch and can be captured into a hipGraph.
+// einsum, a batch of uneven GEMMs). Each becomes a gather-GEMM problem, cut into tiles of one
+// wave each; the tiles of all problems form one list sorted by work (longest first), four to
+// a workgroup, in one launch per wave of items whose outputs do not overlap. Descriptors live
+// in device memory, so executing a plan is a pure kernel launch and can be captured into a
+// hipGraph.
 
 namespace ein {
 
+// One contraction as the wave kernel sees it: C[i,j] = alpha sum_p A[i,p] B[p,j] + beta C[i,j]
+// with element offsets from tables. C's unit stride, if it has one, is along i.
 template <typename T>
-struct GroupedItem {
-    GatherProblem<T> P;
-    int32_t flags; // bit 0: A walks rows (i-fast), bit 1: B walks columns (j-fast)
-    int32_t pad;
+struct WaveItem {
+    T const *A;
+    T const *B;
+    T *C;
+    T alpha, beta;
+    int64_t const *rowA, *rowC, *colB, *colC, *kA, *kB;
+    int64_t kA_in, kB_in; // stride per contraction step where k_mode says so
+    int64_t sA, sC, tB, tC; // strides of a single row digit (i) and column digit (j)
+    int32_t m, n, k;
+    int32_t k_mode; // 2: p * kA_in; 1: kA[p0] + (p - p0) * kA_in within 16 steps from p0; 0: kA[p]
+    int32_t m_lin, n_lin; // offsets of i (j) are i * sA, i * sC (j * tB, j * tC): no table
 };
 
-struct GroupedTile {
-    uint32_t item;
-    uint32_t tile;
+struct WaveTile {
+    int32_t item, tm, tn, pad; // tile (tm, tn) of the item, in units of its wave tile
+    int64_t oa, ob, oc;        // batch offsets
 };
 
-template <typename T, int BM>
-__global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_grouped_kernel(GroupedItem<T> const *__restrict__ items,
-                                                                       GroupedTile const *__restrict__ tiles,
-                                                                       uint32_t ntiles) {
-    constexpr int BN = 64, BK = 16;
-    // the k-major layouts (padded) are the larger ones
-    __shared__ __attribute__((aligned(16))) T As[2 * SlabLayout<T, BM, BK, false, false>::SIZE];
-    __shared__ __attribute__((aligned(16))) T Bs[2 * SlabLayout<T, BN, BK, false, false>::SIZE];
-    static_assert(SlabLayout<T, BM, BK, false, false>::SIZE >= SlabLayout<T, BM, BK, true, false>::SIZE &&
-                      SlabLayout<T, BN, BK, false, false>::SIZE >= SlabLayout<T, BN, BK, true, false>::SIZE,
-                  "LDS sized for the larger layout");
-    for (uint32_t tt = blockIdx.x; tt < ntiles; tt += gridDim.x) {
-        GroupedTile const e           = tiles[tt];
-        GroupedItem<T> const &it      = items[e.item];
-        uint64_t const S              = uint64_t((it.P.k + BK - 1) / BK);
-        switch (it.flags) {
-        case 3: gather_segment<T, BM, BN, BK, false, false, false, false>(it.P, e.tile, 0, S, As, Bs, nullptr); break;
-        case 1: gather_segment<T, BM, BN, BK, false, false, true, false>(it.P, e.tile, 0, S, As, Bs, nullptr); break;
-        case 2: gather_segment<T, BM, BN, BK, true, false, false, false>(it.P, e.tile, 0, S, As, Bs, nullptr); break;
-        default: gather_segment<T, BM, BN, BK, true, false, true, false>(it.P, e.tile, 0, S, As, Bs, nullptr); break;
+// Blocks of 16 rows (columns) in a wave tile: as many as the extent fills, up to most.
+__host__ __device__ __forceinline__ int wave_blocks(int64_t extent, int most) {
+    return extent <= 16 ? 1 : extent <= 32 || most < 4 ? 2 : 4;
+}
+
+// One wave's tile of 16*FM x 16*FN of C. The operands go from global memory straight to the
+// registers that feed the MFMA, 16 contraction steps at a time, the next 16 in flight during
+// the MFMAs: tiles of the small blocks that a grouped plan is made of share little that LDS
+// could hold for them, and without it there is no barrier, no padding to a slab layout, and
+// any alignment takes whole elements. Rows and columns outside the problem read its last one
+// and are not stored; steps beyond k are zeros in both operands. What bounds a plan of many
+// small items is the latency of a tile's first loads, so several waves share a SIMD and only
+// multi-digit indices go through tables. 1024 FP64 GEMMs with extents 4..512 took 1022 us with
+// 64/128 x 64 LDS tiles in a persistent walk, and take 133; 4096 of them 3.24 -> 0.51 ms
+// (FP32 1.20 -> 0.32); 2048 of 32 x 32 x 256 619 -> 53 us; 64 of 384^3 823 -> 198 (36 TFLOP/s).
+template <typename T, int FM, int FN>
+__device__ __forceinline__ void wave_tile(WaveItem<T> const &it, WaveTile const &e, int lane) {
+    int const r  = lane & 15;
+    int const q  = lane >> 4;
+    int const i0 = e.tm * 16 * FM, j0 = e.tn * 16 * FN;
+    int const k  = it.k;
+    T const *pa[FM];
+    T const *pb[FN];
+#pragma unroll
+    for (int a = 0; a < FM; ++a) {
+        int const i = i0 + a * 16 + r;
+        int const ic = i < it.m ? i : it.m - 1;
+        pa[a]        = it.A + e.oa + (it.m_lin ? ic * it.sA : it.rowA[ic]);
+    }
+#pragma unroll
+    for (int b = 0; b < FN; ++b) {
+        int const j = j0 + b * 16 + r;
+        int const jc = j < it.n ? j : it.n - 1;
+        pb[b]        = it.B + e.ob + (it.n_lin ? jc * it.tB : it.colB[jc]);
+    }
+    typename Mfma<T>::acc_t acc[FM][FN];
+#pragma unroll
+    for (int a = 0; a < FM; ++a)
+#pragma unroll
+        for (int b = 0; b < FN; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[a][b][v] = T(0);
+
+    struct Chunk {
+        T a[FM][4], b[FN][4];
+    };
+    // Which of a chunk's 16 steps lane group q feeds to the s-th MFMA does not matter as long as
+    // both operands agree. In a whole chunk it is V consecutive ones, so that an operand
+    // contiguous along k is read 16 bytes at a time (from any element: the hardware takes
+    // 16-byte loads at 4-byte alignment).
+    constexpr int V = 16 / int(sizeof(T));
+    typedef T vec_t __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+    auto load = [&](int k0, Chunk &x) {
+        if (k0 + 16 <= k && it.k_mode != 0) {
+            int64_t const ba = it.k_mode == 2 ? k0 * it.kA_in : it.kA[k0];
+            int64_t const bb = it.k_mode == 2 ? k0 * it.kB_in : it.kB[k0];
+            auto operand = [&](auto const &ptr, int64_t base, int64_t step, auto &out, auto blocks) {
+                constexpr int NBK = decltype(blocks)::value;
+                if (step == 1) {
+#pragma unroll
+                    for (int h = 0; h < 4 / V; ++h)
+#pragma unroll
+                        for (int a = 0; a < NBK; ++a) {
+                            vec_t const t = *reinterpret_cast<vec_t const *>(ptr[a] + base + 4 * V * h + V * q);
+#pragma unroll
+                            for (int v = 0; v < V; ++v) out[a][V * h + v] = t[v];
+                        }
+                } else {
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        int64_t const o = base + (4 * V * (s / V) + V * q + s % V) * step;
+#pragma unroll
+                        for (int a = 0; a < NBK; ++a) out[a][s] = ptr[a][o];
+                    }
+                }
+            };
+            operand(pa, ba, it.kA_in, x.a, std::integral_constant<int, FM>{});
+            operand(pb, bb, it.kB_in, x.b, std::integral_constant<int, FN>{});
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                if (k0 + 4 * s >= k) break;
+                int const p0     = k0 + 4 * s + q;
+                bool const in    = p0 < k;
+                int const p      = in ? p0 : k - 1;
+                int64_t const oa = it.k_mode == 2 ? p * it.kA_in : it.kA[p];
+                int64_t const ob = it.k_mode == 2 ? p * it.kB_in : it.kB[p];
+#pragma unroll
+                for (int a = 0; a < FM; ++a) {
+                    T const t  = pa[a][oa];
+                    x.a[a][s] = in ? t : T(0);
+                }
+#pragma unroll
+                for (int b = 0; b < FN; ++b) {
+                    T const t  = pb[b][ob];
+                    x.b[b][s] = in ? t : T(0);
+                }
+            }
         }
+    };
+    auto multiply = [&](int k0, Chunk const &x) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (k0 + 4 * s >= k) break;
+#pragma unroll
+            for (int a = 0; a < FM; ++a)
+#pragma unroll
+                for (int b = 0; b < FN; ++b) acc[a][b] = Mfma<T>::mma(x.b[b][s], x.a[a][s], acc[a][b]);
+        }
+    };
+    Chunk x, y;
+    load(0, x);
+    for (int k0 = 0; k0 < k; k0 += 32) {
+        if (k0 + 16 < k) load(k0 + 16, y);
+        multiply(k0, x);
+        if (k0 + 16 >= k) break;
+        if (k0 + 32 < k) load(k0 + 32, x);
+        multiply(k0 + 16, y);
+    }
+
+    T *__restrict__ C = it.C + e.oc;
+#pragma unroll
+    for (int a = 0; a < FM; ++a) {
+        int const i = i0 + a * 16 + r;
+        if (i >= it.m) continue;
+        T *ci = C + (it.m_lin ? i * it.sC : it.rowC[i]);
+#pragma unroll
+        for (int b = 0; b < FN; ++b) {
+            int64_t oc[4];
+            T old[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                int const j = j0 + b * 16 + Mfma<T>::row(q, v);
+                int const jc = j < it.n ? j : it.n - 1;
+                oc[v]        = it.n_lin ? jc * it.tC : it.colC[jc];
+                old[v]      = it.beta != T(0) && j < it.n ? ci[oc[v]] : T(0);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (j0 + b * 16 + Mfma<T>::row(q, v) < it.n)
+                    ci[oc[v]] = it.beta != T(0) ? it.alpha * acc[a][b][v] + it.beta * old[v] : it.alpha * acc[a][b][v];
+        }
+    }
+}
+
+// Grouped launch: one tile per wave, in list order (the hardware hands the next workgroup to
+// the next free slot, so the long tiles go first). MOST = 2 or 4 blocks of 16 rows per tile.
+template <typename T, int MOST>
+__global__ __launch_bounds__(GEMM_THREADS, MOST == 2 ? 3 : 2) void grouped_wave_kernel(WaveItem<T> const *__restrict__ items,
+                                                                                        WaveTile const *__restrict__ tiles,
+                                                                                        uint32_t ntiles) {
+    uint32_t const t = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (t >= ntiles) return;
+    int const lane        = threadIdx.x & 63;
+    WaveTile const e      = tiles[t];
+    WaveItem<T> const &it = items[e.item];
+    int const fm = wave_blocks(it.m, MOST), fn = wave_blocks(it.n, 2);
+    if constexpr (MOST == 4) {
+        if (fm == 4) {
+            if (fn == 2)
+                wave_tile<T, 4, 2>(it, e, lane);
+            else
+                wave_tile<T, 4, 1>(it, e, lane);
+            return;
+        }
+    }
+    if (fm == 2) {
+        if (fn == 2)
+            wave_tile<T, 2, 2>(it, e, lane);
+        else
+            wave_tile<T, 2, 1>(it, e, lane);
+    } else {
+        if (fn == 2)
+            wave_tile<T, 1, 2>(it, e, lane);
+        else
+            wave_tile<T, 1, 1>(it, e, lane);
     }
 }
 
@@ -1129,8 +1294,8 @@ struct PreScale {
 struct GroupedWave {
     std::vector<PreScale> prescale;        // C scales that must precede this wave's tiles
     std::vector<ein_contraction_item> large; // items that fill the GPU alone: regular dispatch
-    void *d_items[2] = {nullptr, nullptr}; // per tile height (64, 128)
-    void *d_tiles[2] = {nullptr, nullptr};
+    void *d_items    = nullptr;
+    void *d_tiles[2] = {nullptr, nullptr}; // per tile height (2 or 4 blocks of 16 rows a wave)
     void *d_tables   = nullptr;            // offset tables of the wave's items
     uint32_t ntiles[2] = {0, 0};
 };
@@ -1143,18 +1308,15 @@ void free_wave(GroupedWave &w, hipStream_t stream = nullptr, bool known = false)
         if (known) (void)ein_free_async(p, stream);
         else (void)ein_free(p);
     };
-    for (int v = 0; v < 2; ++v) {
-        release(w.d_items[v]);
-        release(w.d_tiles[v]);
-        w.d_items[v] = w.d_tiles[v] = nullptr;
+    for (void **p : {&w.d_items, &w.d_tiles[0], &w.d_tiles[1], &w.d_tables}) {
+        release(*p);
+        *p = nullptr;
     }
-    release(w.d_tables);
-    w.d_tables = nullptr;
 }
 
 struct GroupedPlan {
     int elem = 8;
-    int bm_index = 0; // 0: 64-row tiles, 1: 128-row tiles
+    int bm_index = 0; // 0: 32-row wave tiles (64 rows a workgroup), 1: 64-row (128)
     bool tuned = false;
     std::vector<GroupedWave> waves;
     std::vector<ein_contraction_item> items; // host copy (for the autotuner)
@@ -1197,10 +1359,18 @@ ByteRange range_of(ein_tensor_desc const &d, void const *p, size_t elem) {
     return {base + uintptr_t(lo * int64_t(elem)), base + uintptr_t((hi + 1) * int64_t(elem))};
 }
 
-// Analyse one item into a gather problem (MFMA path for every size). kind: 0 = tiles to
-// run, 1 = only a scale of C, 2 = nothing to do.
+// One item: its problem with the index groups that its tables are built from.
 template <typename T>
-int build_item(ein_contraction_item const &in, GroupedItem<T> (&out)[2], int &kind, bool &c_repeats) {
+struct BuiltItem {
+    WaveItem<T> w;
+    IndexGroup gm, gn, gk, gb; // (A, C), (B, C), (A, B) and (A, B, C) strides
+    int64_t batch;
+};
+
+// Analyse one item (MFMA path for every size). kind: 0 = tiles to run, 1 = only a scale of C,
+// 2 = nothing to do.
+template <typename T>
+int build_item(ein_contraction_item const &in, BuiltItem<T> &out, int &kind, bool &c_repeats) {
     ContractionAnalysis an;
     EIN_TRY(analyse_contraction(in.C, in.A, in.B, an));
     c_repeats = an.c_repeats;
@@ -1231,41 +1401,57 @@ int build_item(ein_contraction_item const &in, GroupedItem<T> (&out)[2], int &ki
         kind = 1;
         return EIN_SUCCESS;
     }
-    int64_t const M = total_of(vm), N = total_of(vn), K = total_of(vk), NB = total_of(vb);
+    int64_t M = total_of(vm), N = total_of(vn);
+    int64_t const K = total_of(vk), NB = total_of(vb);
     if (M >= (int64_t{1} << 31) || N >= (int64_t{1} << 31) || K >= (int64_t{1} << 31) || NB >= (int64_t{1} << 31))
         return fail(EIN_ERROR_UNSUPPORTED, "grouped contraction: index range above 2^31");
+    // the lanes of a wave run along i when C is read and written: the side that holds C's
+    // unit stride becomes A
+    auto unit_in_c = [](std::vector<Digit> const &v) {
+        for (auto const &d : v)
+            if (std::llabs(d.s[1]) == 1) return true;
+        return false;
+    };
+    bool const swap = unit_in_c(vn) && !unit_in_c(vm);
+    T const *pa = static_cast<T const *>(in.a), *pb = static_cast<T const *>(in.b);
+    if (swap) {
+        std::swap(vm, vn);
+        std::swap(M, N);
+        std::swap(pa, pb);
+        for (auto &d : vk) std::swap(d.s[0], d.s[1]);
+        for (auto &d : vb) std::swap(d.s[0], d.s[1]);
+    }
     auto gm = order_and_fold(vm, 2, 0, 1);
     auto gn = order_and_fold(vn, 2, 0, 1);
     bool const a_i_fast = !gm.empty() && std::llabs(gm.back().s[0]) == 1;
     auto gk = a_i_fast ? order_and_fold(vk, 2, 1, 0) : order_and_fold(vk, 2, 0, 1);
-    bool const b_j_fast = (!gn.empty() && std::llabs(gn.back().s[0]) == 1) ||
-                          !(!gk.empty() && std::llabs(gk.back().s[1]) == 1);
-    bool const a_fast = a_i_fast || !(!gk.empty() && std::llabs(gk.back().s[0]) == 1);
     auto gbv = order_and_fold(vb, 3, 2, 0);
-    GatherProblem<T> P{};
-    EIN_TRY(fill_group(P.gm, gm, 2));
-    EIN_TRY(fill_group(P.gn, gn, 2));
-    EIN_TRY(fill_group(P.gk, gk, 2));
-    EIN_TRY(fill_group(P.gb, gbv, 3));
-    set_k_affine(P, gk);
-    P.m = M;
-    P.n = N;
-    P.k = K;
-    P.batch = NB;
-    P.A = static_cast<T const *>(in.a);
-    P.B = static_cast<T const *>(in.b);
-    P.C = static_cast<T *>(in.c);
-    P.alpha = T(in.ab_prefactor);
-    P.beta = c_repeats ? T(1) : T(in.c_prefactor);
-    P.partial = nullptr;
-    int const bms[2] = {64, 128};
-    for (int v = 0; v < 2; ++v) {
-        out[v].P = P;
-        out[v].P.tiles_m = uint32_t(ceil_div(M, bms[v]));
-        out[v].P.tiles_n = uint32_t(ceil_div(N, 64));
-        out[v].flags = (a_fast ? 1 : 0) | (b_j_fast ? 2 : 0);
-        out[v].pad = 0;
-    }
+    EIN_TRY(fill_group(out.gm, gm, 2));
+    EIN_TRY(fill_group(out.gn, gn, 2));
+    EIN_TRY(fill_group(out.gk, gk, 2));
+    EIN_TRY(fill_group(out.gb, gbv, 3));
+    out.batch       = NB;
+    WaveItem<T> &w  = out.w;
+    w        = WaveItem<T>{};
+    w.A      = pa;
+    w.B      = pb;
+    w.C      = static_cast<T *>(in.c);
+    w.alpha  = T(in.ab_prefactor);
+    w.beta   = c_repeats ? T(1) : T(in.c_prefactor);
+    w.m      = int32_t(M);
+    w.n      = int32_t(N);
+    w.k      = int32_t(K);
+    // one digit: affine over all of k. Otherwise affine within 16 steps where the innermost
+    // digit's extent is a multiple of 16 (chunks start at multiples of 16)
+    w.k_mode = gk.size() <= 1 ? 2 : gk.back().e % 16 == 0 ? 1 : 0;
+    w.kA_in  = gk.empty() ? 0 : gk.back().s[0];
+    w.kB_in  = gk.empty() ? 0 : gk.back().s[1];
+    w.m_lin  = gm.size() <= 1;
+    w.n_lin  = gn.size() <= 1;
+    w.sA     = gm.empty() ? 0 : gm.back().s[0];
+    w.sC     = gm.empty() ? 0 : gm.back().s[1];
+    w.tB     = gn.empty() ? 0 : gn.back().s[0];
+    w.tC     = gn.empty() ? 0 : gn.back().s[1];
     return EIN_SUCCESS;
 }
 
@@ -1279,7 +1465,7 @@ template <typename T>
 int plan_create(ein_contraction_item const *items, int count, GroupedPlan &plan,
                 std::vector<int> const *forced_waves = nullptr) {
     plan.elem = int(sizeof(T));
-    std::vector<std::vector<GroupedItem<T>>> wave_items[2];
+    std::vector<std::vector<BuiltItem<T>>> wave_items;
     struct Placed {
         ByteRange out, in_a, in_b;
         int wave;
@@ -1287,7 +1473,7 @@ int plan_create(ein_contraction_item const *items, int count, GroupedPlan &plan,
     std::vector<Placed> placed;
     size_t const eb = sizeof(T);
     for (int i = 0; i < count; ++i) {
-        GroupedItem<T> gi[2]{};
+        BuiltItem<T> gi{};
         int kind = 0;
         bool rep = false;
         EIN_TRY(build_item<T>(items[i], gi, kind, rep));
@@ -1306,100 +1492,129 @@ int plan_create(ein_contraction_item const *items, int count, GroupedPlan &plan,
         size_t const w = size_t(me.wave);
         while (w >= plan.waves.size()) {
             plan.waves.emplace_back();
-            wave_items[0].emplace_back();
-            wave_items[1].emplace_back();
+            wave_items.emplace_back();
         }
         placed.push_back(me);
         plan.items.push_back(items[i]);
         plan.wave_of.push_back(me.wave);
-        // Items with 16 or more 128 x 128 tiles keep their own tuned kernels (wide DMA,
-        // 128 x 128 tiles, stream-K over all CUs), and so do items with a long contraction
-        // (k >= 2048), whose few tiles would each run k/16 slabs on one CU here while
-        // stream-K splits them over the GPU. The persistent kernel takes the many small,
-        // short items, for which one launch each would cost more than the work.
-        bool const big_tiles = kind == 0 && gi[0].P.m >= 128 && gi[0].P.n >= 128 &&
-                               ceil_div(gi[0].P.m, 128) * ceil_div(gi[0].P.n, 128) * gi[0].P.batch >= 16;
-        if (kind == 0 && (big_tiles || gi[0].P.k >= 2048)) {
+        // Items with 16 or more 128 x 128 tiles and 1 GFLOP keep their own tuned kernels (LDS
+        // tiles, stream-K over all CUs), and so do items with a long contraction (k >= 2048),
+        // whose few tiles would each run k/16 chunks on one wave here while stream-K splits
+        // them over the GPU. Smaller ones would leave most of the GPU idle in a launch of their
+        // own: with every 16-tile item launched alone, 1024 GEMMs with extents 4..512 (three
+        // such items) took 192 us against 133, and the W intermediates of 8 irreps 3.35 ms
+        // against 2.84 (3.00 with the line at 0.3 GFLOP, 2.85 at 3).
+        bool const big_tiles = kind == 0 && gi.w.m >= 128 && gi.w.n >= 128 &&
+                               ceil_div(gi.w.m, 128) * ceil_div(gi.w.n, 128) * gi.batch >= 16 &&
+                               2.0 * gi.w.m * gi.w.n * gi.w.k * gi.batch >= 1e9;
+        if (kind == 0 && (big_tiles || gi.w.k >= 2048)) {
             plan.waves[w].large.push_back(items[i]);
             continue;
         }
         if (kind == 1 || rep) plan.waves[w].prescale.push_back({items[i].C, items[i].c, items[i].c_prefactor});
         if (kind == 1) continue;
-        wave_items[0][w].push_back(gi[0]);
-        wave_items[1][w].push_back(gi[1]);
+        wave_items[w].push_back(gi);
     }
     for (size_t w = 0; w < plan.waves.size(); ++w) {
-        // offset tables of the wave's items (shared by both tile heights)
+        auto &its       = wave_items[w];
+        GroupedWave &gw = plan.waves[w];
+        // offset tables of the wave's items: [rowA | rowC | colB | colC | kA | kB] each
         {
             size_t total = 0;
-            for (auto const &it : wave_items[0][w]) total += gather_table_entries(it.P.m, it.P.n, it.P.k);
+            for (auto const &x : its) total += gather_table_entries(x.w.m, x.w.n, x.w.k);
             std::vector<int64_t> host(std::max<size_t>(total, 1));
-            EIN_TRY(ein_malloc(&plan.waves[w].d_tables, std::max<size_t>(total * sizeof(int64_t), 256)));
-            int64_t *dev = static_cast<int64_t *>(plan.waves[w].d_tables);
+            EIN_TRY(ein_malloc(&gw.d_tables, std::max<size_t>(total * sizeof(int64_t), 256)));
+            int64_t *dev = static_cast<int64_t *>(gw.d_tables);
             size_t at = 0;
-            for (size_t q = 0; q < wave_items[0][w].size(); ++q) {
-                GatherProblem<T> &P0 = wave_items[0][w][q].P;
-                int64_t *h           = host.data() + at;
-                host_offsets(P0.gm, P0.m, h, h + P0.m);
-                host_offsets(P0.gn, P0.n, h + 2 * P0.m, h + 2 * P0.m + P0.n);
-                host_offsets(P0.gk, P0.k, h + 2 * (P0.m + P0.n), h + 2 * (P0.m + P0.n) + P0.k);
-                set_tables(P0, dev + at);
-                set_tables(wave_items[1][w][q].P, dev + at);
-                at += gather_table_entries(P0.m, P0.n, P0.k);
+            for (auto &x : its) {
+                int64_t const m = x.w.m, n = x.w.n, k = x.w.k;
+                int64_t *h      = host.data() + at;
+                host_offsets(x.gm, m, h, h + m);
+                host_offsets(x.gn, n, h + 2 * m, h + 2 * m + n);
+                host_offsets(x.gk, k, h + 2 * (m + n), h + 2 * (m + n) + k);
+                int64_t const *t = dev + at;
+                x.w.rowA = t;
+                x.w.rowC = t + m;
+                x.w.colB = t + 2 * m;
+                x.w.colC = t + 2 * m + n;
+                x.w.kA   = t + 2 * (m + n);
+                x.w.kB   = t + 2 * (m + n) + k;
+                at += gather_table_entries(m, n, k);
             }
             if (total) EIN_HIP_CHECK(hipMemcpy(dev, host.data(), total * sizeof(int64_t), hipMemcpyHostToDevice));
         }
+        std::vector<WaveItem<T>> dev_items;
+        for (auto const &x : its) dev_items.push_back(x.w);
+        size_t const ib = dev_items.size() * sizeof(WaveItem<T>);
+        EIN_TRY(ein_malloc(&gw.d_items, std::max<size_t>(ib, 256)));
+        if (ib) EIN_HIP_CHECK(hipMemcpy(gw.d_items, dev_items.data(), ib, hipMemcpyHostToDevice));
         for (int v = 0; v < 2; ++v) {
-            auto const &its = wave_items[v][w];
-            std::vector<GroupedTile> tl;
-            std::vector<int64_t> cost;
+            struct Listed {
+                int64_t cost;
+                WaveTile t;
+            };
+            std::vector<Listed> tl;
             for (size_t q = 0; q < its.size(); ++q) {
-                uint64_t nt = uint64_t(its[q].P.tiles_m) * its[q].P.tiles_n * uint64_t(its[q].P.batch);
-                if (nt > 0xffffffffu) return fail(EIN_ERROR_UNSUPPORTED, "grouped contraction: too many tiles");
-                for (uint64_t t = 0; t < nt; ++t) {
-                    tl.push_back({uint32_t(q), uint32_t(t)});
-                    cost.push_back(its[q].P.k);
+                auto const &x    = its[q];
+                int const fm     = wave_blocks(x.w.m, v == 0 ? 2 : 4), fn = wave_blocks(x.w.n, 2);
+                int64_t const tm = ceil_div(x.w.m, 16 * fm), tn = ceil_div(x.w.n, 16 * fn);
+                if (double(tm) * double(tn) * double(x.batch) + double(tl.size()) > 4294967295.0)
+                    return fail(EIN_ERROR_UNSUPPORTED, "grouped contraction: too many tiles");
+                int64_t const cost = ceil_div(x.w.k, 16) * fm * fn;
+                // 2 x 2 neighbours together: the four waves of a workgroup share their loads
+                for (int64_t z = 0; z < x.batch; ++z) {
+                    WaveTile t{};
+                    t.item = int32_t(q);
+                    uint64_t idx = uint64_t(z);
+                    for (int d = x.gb.n - 1; d >= 0; --d) {
+                        int64_t const digit = int64_t(idx % x.gb.ext[d]);
+                        idx /= x.gb.ext[d];
+                        t.oa += digit * x.gb.s[0][d];
+                        t.ob += digit * x.gb.s[1][d];
+                        t.oc += digit * x.gb.s[2][d];
+                    }
+                    for (int64_t jn = 0; jn < tn; jn += 2)
+                        for (int64_t im = 0; im < tm; im += 2)
+                            for (int64_t y = jn; y < std::min(jn + 2, tn); ++y)
+                                for (int64_t u = im; u < std::min(im + 2, tm); ++u) {
+                                    t.tm = int32_t(u);
+                                    t.tn = int32_t(y);
+                                    tl.push_back({cost, t});
+                                }
                 }
             }
-            // longest contraction first (LPT over a fixed-stride persistent walk)
-            std::vector<size_t> order(tl.size());
-            for (size_t z = 0; z < order.size(); ++z) order[z] = z;
-            std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return cost[x] > cost[y]; });
-            std::vector<GroupedTile> sorted(tl.size());
-            for (size_t z = 0; z < order.size(); ++z) sorted[z] = tl[order[z]];
-            size_t ib = its.size() * sizeof(GroupedItem<T>), tb = sorted.size() * sizeof(GroupedTile);
-            EIN_TRY(ein_malloc(&plan.waves[w].d_items[v], std::max<size_t>(ib, 256)));
-            EIN_TRY(ein_malloc(&plan.waves[w].d_tiles[v], std::max<size_t>(tb, 256)));
-            if (ib) EIN_HIP_CHECK(hipMemcpy(plan.waves[w].d_items[v], its.data(), ib, hipMemcpyHostToDevice));
-            if (tb) EIN_HIP_CHECK(hipMemcpy(plan.waves[w].d_tiles[v], sorted.data(), tb, hipMemcpyHostToDevice));
-            plan.waves[w].ntiles[v] = uint32_t(sorted.size());
+            // longest first
+            std::stable_sort(tl.begin(), tl.end(), [](Listed const &x, Listed const &y) { return x.cost > y.cost; });
+            std::vector<WaveTile> sorted;
+            sorted.reserve(tl.size());
+            for (auto const &x : tl) sorted.push_back(x.t);
+            size_t const tb = sorted.size() * sizeof(WaveTile);
+            EIN_TRY(ein_malloc(&gw.d_tiles[v], std::max<size_t>(tb, 256)));
+            if (tb) EIN_HIP_CHECK(hipMemcpy(gw.d_tiles[v], sorted.data(), tb, hipMemcpyHostToDevice));
+            gw.ntiles[v] = uint32_t(sorted.size());
             plan.tiles_total[v] += int64_t(sorted.size());
         }
     }
-    // default tile height: 128 rows only when it still gives >= 2 tiles per resident slot
-    plan.bm_index = plan.tiles_total[1] >= int64_t(num_cus()) * 4 ? 1 : 0;
+    // The default is 32-row tiles; the autotuner may pick 64-row ones. 1024 GEMMs with extents
+    // 4..512 run in 133 us with 32 rows and 141 with 64; 64 of 511 x 127 x 511 in 162 and 117.
+    plan.bm_index = 0;
     return EIN_SUCCESS;
 }
 
 template <typename T>
 int plan_launch(GroupedPlan const &plan, int bm_index, hipStream_t stream) {
-    void const *k128 = reinterpret_cast<void const *>(&gemm_grouped_kernel<T, 128>);
-    void const *k64  = reinterpret_cast<void const *>(&gemm_grouped_kernel<T, 64>);
-    uint32_t const slots =
-        uint32_t(num_cus()) * uint32_t(resident_blocks(bm_index == 1 ? k128 : k64, GEMM_THREADS));
     for (auto const &w : plan.waves) {
         for (auto const &ps : w.prescale)
             EIN_TRY(tensor_scale<T>(ps.C, static_cast<T *>(ps.c), T(ps.factor), stream));
-        uint32_t nt = w.ntiles[bm_index];
+        uint32_t const nt = w.ntiles[bm_index];
         if (nt != 0) {
-            uint32_t grid = nt < slots ? nt : slots;
+            uint32_t const grid = uint32_t(ceil_div(nt, 4));
+            auto const *items   = static_cast<WaveItem<T> const *>(w.d_items);
+            auto const *tiles   = static_cast<WaveTile const *>(w.d_tiles[bm_index]);
             if (bm_index == 1)
-                gemm_grouped_kernel<T, 128><<<grid, GEMM_THREADS, 0, stream>>>(
-                    static_cast<GroupedItem<T> const *>(w.d_items[1]), static_cast<GroupedTile const *>(w.d_tiles[1]),
-                    nt);
+                grouped_wave_kernel<T, 4><<<grid, GEMM_THREADS, 0, stream>>>(items, tiles, nt);
             else
-                gemm_grouped_kernel<T, 64><<<grid, GEMM_THREADS, 0, stream>>>(
-                    static_cast<GroupedItem<T> const *>(w.d_items[0]), static_cast<GroupedTile const *>(w.d_tiles[0]), nt);
+                grouped_wave_kernel<T, 2><<<grid, GEMM_THREADS, 0, stream>>>(items, tiles, nt);
             EIN_LAUNCH_CHECK();
         }
         for (auto const &it : w.large)
