@@ -49,6 +49,21 @@ def stream_handle(stream: torch.cuda.Stream | None = None) -> ctypes.c_void_p:
     return ctypes.c_void_p(s.cuda_stream)
 
 
+# The raw handle of the current stream, without the Stream object around it (2.9 us a call).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _current_stream() -> int:
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
+
+
+def _on(stream: torch.cuda.Stream | None):
+    """The context of ``stream``; nothing to enter when it is the current one already."""
+    return contextlib.nullcontext() if stream is None else torch.cuda.stream(stream)
+
+
 def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr())
 
@@ -122,14 +137,33 @@ def _as_device(x, write: bool):
     raise TypeError(f"unsupported operand type {type(x).__name__}")
 
 
+# Descriptors by their content (labels, extents, strides): a program meets the same few again
+# and again, and filling a ctypes structure takes over a microsecond. Read only once made.
+_descs: dict = {}
+_DESCS_KEPT = 1024
+
+
 def _desc(t: torch.Tensor, idx: str):
-    if t.dim() != len(idx):
-        raise RankError(f"rank of tensor ({t.dim()}) does not match index string {idx!r}")
-    return make_desc(idx, t.shape, t.stride())
+    key = (idx, t.shape, t.stride())
+    d = _descs.get(key)
+    if d is None:
+        if t.dim() != len(idx):
+            raise RankError(f"rank of tensor ({t.dim()}) does not match index string {idx!r}")
+        d = make_desc(idx, t.shape, t.stride())
+        if len(_descs) >= _DESCS_KEPT:
+            _descs.clear()
+        _descs[key] = d
+    return d
+
+
+_fns: dict = {}
 
 
 def _fn(name: str, dtype: torch.dtype):
-    return getattr(lib, f"{name}_{'f64' if dtype == torch.float64 else 'f32'}")
+    f = _fns.get((name, dtype))
+    if f is None:
+        f = _fns[name, dtype] = getattr(lib, f"{name}_{'f64' if dtype == torch.float64 else 'f32'}")
+    return f
 
 
 def _labels_only_desc(idx: str):
@@ -172,11 +206,11 @@ class EinsumGenericPlan:
         # every torch op of the call (staging copies, temporaries, the copy back) runs on the
         # kernel's stream, so they are ordered with it and the caching allocator reuses the
         # temporaries only after the kernel
-        with torch.cuda.stream(stream):
+        with _on(stream):
             self._execute_one(C_prefactor, C, AB_prefactor, A, B, split, slice_type)
 
     def _execute_one(self, C_prefactor, C, AB_prefactor, A, B, split, slice_type) -> None:
-        stream = None  # the current stream, set by execute()
+        # on the current stream, set by execute()
         dC, finC = _as_device(C, write=True)
         dA, _ = _as_device(A, write=False)
         dB, _ = _as_device(B, write=False)
@@ -197,14 +231,15 @@ class EinsumGenericPlan:
             if dtype != torch.float64:
                 raise TypeError("split precision applies to float64 operands")
             st = _slice_code(slice_type)
-            status = lib.ein_einsum_split_f64(_split_count(split), st, float(C_prefactor), ctypes.byref(cd), _ptr(dC),
-                                              float(AB_prefactor), ctypes.byref(ad), _ptr(dA), ctypes.byref(bd), _ptr(dB),
-                                              ctypes.byref(used), stream_handle(stream))
+            status = lib.ein_einsum_split_f64(_split_count(split), st, C_prefactor, ctypes.byref(cd), dC.data_ptr(),
+                                              AB_prefactor, ctypes.byref(ad), dA.data_ptr(), ctypes.byref(bd),
+                                              dB.data_ptr(), ctypes.byref(used), _current_stream())
         else:
-            fn = _fn("ein_einsum_execute", dtype)
-            status = fn(self.algorithm, float(C_prefactor), ctypes.byref(cd), _ptr(dC), float(AB_prefactor),
-                        ctypes.byref(ad), _ptr(dA), ctypes.byref(bd), _ptr(dB), ctypes.byref(used), stream_handle(stream))
-        check(status, f"einsum {self.C_indices} <- {self.A_indices},{self.B_indices}")
+            status = _fn("ein_einsum_execute", dtype)(self.algorithm, C_prefactor, ctypes.byref(cd), dC.data_ptr(),
+                                                      AB_prefactor, ctypes.byref(ad), dA.data_ptr(), ctypes.byref(bd),
+                                                      dB.data_ptr(), ctypes.byref(used), _current_stream())
+        if status != _lib.EIN_SUCCESS:
+            check(status, f"einsum {self.C_indices} <- {self.A_indices},{self.B_indices}")
         self.last_algorithm = used.value
         if finC is not None:
             torch.cuda.current_stream().synchronize()
@@ -328,12 +363,27 @@ def permute(C_prefactor: float, C_indices: str, C: torch.Tensor, A_prefactor: fl
     ``permute(beta, Indices{...}, &C, alpha, Indices{...}, A)``, Permute.hpp:330-407)."""
     if sorted(C_indices) != sorted(A_indices) or len(set(A_indices)) != len(A_indices):
         raise ValueError(f"permute: {C_indices!r} is not a permutation of {A_indices!r}")
-    with torch.cuda.stream(stream):
+    with _on(stream):
         _permute_one(C_prefactor, C_indices, C, A_prefactor, A_indices, A)
 
 
+class _Arrays(dict):
+    """ctypes array types by length (making the type anew takes longer than an instance)."""
+
+    def __init__(self, element):
+        super().__init__()
+        self.element = element
+
+    def __missing__(self, r):
+        self[r] = self.element * max(r, 1)
+        return self[r]
+
+
+_I64, _I32 = _Arrays(ctypes.c_int64), _Arrays(ctypes.c_int32)
+
+
 def _permute_one(C_prefactor, C_indices, C, A_prefactor, A_indices, A) -> None:
-    stream = None  # the current stream, set by permute()
+    # on the current stream, set by permute()
     dC, finC = _as_device(C, write=True)
     dA, _ = _as_device(A, write=False)
     if dC.dtype == dA.dtype and dC.dtype in _COMPLEX:
@@ -364,10 +414,9 @@ def _permute_one(C_prefactor, C_indices, C, A_prefactor, A_indices, A) -> None:
     for i in range(r):
         if dC.shape[i] != dA.shape[perm[i]]:
             raise DimensionError("permute: extents do not match")
-    I64 = ctypes.c_int64 * max(r, 1)
-    I32 = ctypes.c_int32 * max(r, 1)
-    status = _fn("ein_permute", dC.dtype)(r, I64(*dA.shape), I32(*perm), float(A_prefactor), _ptr(dA), I64(*dA.stride()),
-                                          float(C_prefactor), _ptr(dC), I64(*dC.stride()), stream_handle(stream))
+    I64, I32 = _I64[r], _I32[r]
+    status = _fn("ein_permute", dC.dtype)(r, I64(*dA.shape), I32(*perm), A_prefactor, dA.data_ptr(), I64(*dA.stride()),
+                                          C_prefactor, dC.data_ptr(), I64(*dC.stride()), _current_stream())
     check(status, "permute")
     if finC is not None:
         torch.cuda.current_stream().synchronize()
@@ -390,7 +439,7 @@ def syev(A: torch.Tensor, W: torch.Tensor, compute_vectors: bool = True, stream=
     orthonormal eigenvectors as columns (``A[:, j]`` belongs to ``W[j]``) and W with the
     eigenvalues in ascending order. Returns the device ``info`` tensor; with ``check_info``
     it is read (a synchronisation) and a failure to converge raises, as in the reference."""
-    with torch.cuda.stream(stream):
+    with _on(stream):
         return _syev_body(A, W, compute_vectors, check_info)
 
 
@@ -403,7 +452,7 @@ def _syev_body(A, W, compute_vectors, check_info):
         raise DimensionError("syev: W must have n entries")
     if W.dtype != A.dtype or not W.is_contiguous():
         raise TypeError("syev: W must be a contiguous vector of A's dtype")
-    info = torch.zeros((), dtype=torch.int32, device=A.device)
+    info = torch.empty((), dtype=torch.int32, device=A.device)  # the solver writes it, whatever n
     job = b"V" if compute_vectors else b"N"
     fn = _fn("ein_syev", A.dtype)
     if A.stride(0) == 1 and A.stride(1) >= max(1, n):
@@ -459,7 +508,7 @@ def _gesv_body(A, B, check_info):
 def gemm(transA: str, transB: str, alpha: float, A: torch.Tensor, B: torch.Tensor, beta: float, C: torch.Tensor,
          stream=None) -> None:
     """Row-major C = alpha*op(A) op(B) + beta*C on 2-D tensors (linear_algebra::gemm)."""
-    with torch.cuda.stream(stream):
+    with _on(stream):
         return _gemm_body(transA, transB, alpha, A, B, beta, C)
 
 
@@ -542,7 +591,7 @@ def fock_jk(g: torch.Tensor, D: torch.Tensor, F: torch.Tensor, alpha_j: float = 
     Equals the reference's pair of calls
     ``einsum(1, "ij", F, alpha_j, "kl", D, "ijkl", g)`` and ``einsum(1, "ij", F, alpha_k, "kl", D, "ikjl", g)``
     (QChemTests.cpp:299-304) after ``F *= beta``; the defaults give G = 2J - K. n <= 128."""
-    with torch.cuda.stream(stream):
+    with _on(stream):
         n = int(g.shape[0]) if g.dim() == 4 else -1
         if g.dim() != 4 or tuple(g.shape) != (n,) * 4 or not g.is_contiguous():
             raise ValueError("fock_jk: g must be a contiguous n x n x n x n tensor")
