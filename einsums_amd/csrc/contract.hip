@@ -869,10 +869,9 @@ int contract_generic(T c_prefactor, ein_tensor_desc const &C, T *c, T ab_prefact
         uint64_t tiles   = uint64_t(P.tiles_m) * P.tiles_n * uint64_t(NB);
         if (tiles > 0x7fffffffu) return fail(EIN_ERROR_UNSUPPORTED, "contraction tile grid too large");
         OperandStaging sa{!a_fast, false}, sb{!b_j_fast, false};
-        constexpr int EW = int(sizeof(T)) / 4;
-        sa.wide = a_fast ? (bm * EW >= 256 && gather_wide_ok<T>(gm, 0, gk, 0, gbv, 0, a))
+        sa.wide = a_fast ? (kmajor_wide<T>(bm) && gather_wide_ok<T>(gm, 0, gk, 0, gbv, 0, a))
                          : gather_wide_ok<T>(gk, 0, gm, 0, gbv, 0, a);
-        sb.wide = b_j_fast ? (bn * EW >= 256 && gather_wide_ok<T>(gn, 0, gk, 1, gbv, 1, b))
+        sb.wide = b_j_fast ? (kmajor_wide<T>(bn) && gather_wide_ok<T>(gn, 0, gk, 1, gbv, 1, b))
                            : gather_wide_ok<T>(gk, 1, gn, 0, gbv, 1, b);
         void const *kern = bm == 128 && bn == 128 ? gather_kernel_for<T, 128, 128>(sa, sb)
                            : bm == 128            ? gather_kernel_for<T, 128, 64>(sa, sb)

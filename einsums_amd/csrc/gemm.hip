@@ -351,8 +351,17 @@ TuneKey tune_key(GemmProblem<T> const &P) {
 // workgroups per CU the schedule plans for (all that fit, or one).
 // krow_both: both operands contiguous along k (row-major LDS staging), the case the 96 x 96
 // tile is built for (576 = 6 x 96: the Wmnij GEMM at o=24 has no ragged tiles).
-std::vector<GemmConfig> tune_candidates(bool krow_both) {
+// fp32: adds the 256 x 128 tile, which only FP32's accumulators leave registers for.
+std::vector<GemmConfig> tune_candidates(bool krow_both, bool fp32) {
     std::vector<GemmConfig> c;
+    if (fp32)
+        for (int dp : {0, 1}) {
+            GemmConfig g;
+            g.bm            = 256;
+            g.bn            = 128;
+            g.data_parallel = dp;
+            c.push_back(g);
+        }
     if (krow_both)
         for (int dp : {0, 1, 2})
             for (int bpc : {0, 1}) {
@@ -418,7 +427,7 @@ int tune_gemm(GemmProblem<T> const &P, hipStream_t stream, GemmConfig *best) {
     Q.c_sn           = P.m;
     Q.c_sb           = P.m * P.n;
     Q.beta           = P.beta;
-    std::vector<GemmConfig> const cands = tune_candidates(krow_both(P));
+    std::vector<GemmConfig> const cands = tune_candidates(krow_both(P), sizeof(T) == 4);
     std::vector<float> best_of(cands.size(), 0.f);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int st = EIN_SUCCESS;
@@ -497,7 +506,7 @@ int gemm_strided_impl(GemmProblem<T> P, GemmConfig const *force, hipStream_t str
             if (ws_bytes != nullptr) {
                 // an untuned key in tuning mode may run any candidate: report the largest need
                 size_t most = 0;
-                for (GemmConfig const &c : tune_candidates(krow_both(P))) {
+                for (GemmConfig const &c : tune_candidates(krow_both(P), sizeof(T) == 4)) {
                     size_t b = 0;
                     EIN_TRY(gemm_strided_impl<T>(P, &c, stream, &b));
                     most = std::max(most, b);
@@ -522,8 +531,20 @@ int gemm_strided_impl(GemmProblem<T> P, GemmConfig const *force, hipStream_t str
         bool const b_krow = choose_staging<T>(64, P.b_sn, P.b_sk, P.b_sb, P.batch, P.n, P.k, P.B).krow;
         if (a_krow && b_krow) cfg.bm = 64;
     }
+    if (sizeof(T) == 4 && !force && cfg.bm == 128 && cfg.bn == 128 &&
+        ceil_div(P.m, 256) * ceil_div(P.n, 128) * P.batch >= 2 * int64_t(num_cus())) {
+        // FP32 slabs of 128 x 128 are half as long in time as FP64's, and what they stage per
+        // MFMA is what holds them back (without the staging 140 TFLOP/s, with it 119): from two
+        // rounds of 256 x 128 tiles on, a wave of 128 x 64 stages a quarter less. 4096^3 NN
+        // 1155 -> 1066 us, NT 1128 -> 1077, TN 1060 -> 1037; with fewer tiles the last round costs
+        // more than that (3000^3, 288 tiles: TN 453 -> 474; 1536^3, 72 tiles: NN 81 -> 88).
+        cfg.bm            = 256;
+        cfg.blocks_per_cu = 0;
+    }
     P.force_dp     = cfg.data_parallel;
     constexpr int BK = 16;
+    if constexpr (sizeof(T) == 4)
+        if (cfg.bm == 256) return launch_dense<T, 256, 128, BK>(P, cfg.blocks_per_cu, stream, ws_bytes);
     if (cfg.bm == 96 && cfg.bn == 96) {
         if (!krow_both(P))
             return fail(EIN_ERROR_UNSUPPORTED, "gemm: 96 x 96 tiles need FP64 operands contiguous along k");
@@ -802,7 +823,8 @@ int ein_gemm_tuning_load(const char *path) {
         long long m, n, k, b;
         if (std::sscanf(line, "%d %lld %lld %lld %lld %d %d : %d %d %d %d", &eb, &m, &n, &k, &b, &ak, &bk, &bm, &bn, &dp,
                         &bpc) != 11 ||
-            (eb != 4 && eb != 8) || (bm != 64 && bm != 96 && bm != 128) || (bn != 64 && bn != 96 && bn != 128) || (bm == 96) != (bn == 96) ||
+            (eb != 4 && eb != 8) || (bm != 64 && bm != 96 && bm != 128 && (bm != 256 || eb != 4 || bn != 128)) ||
+            (bn != 64 && bn != 96 && bn != 128) || (bm == 96) != (bn == 96) ||
             dp < 0 || dp > 2 || bpc < 0 ||
             m <= 0 || n <= 0 || k <= 0 || b <= 0) {
             std::fclose(f);

@@ -12,7 +12,11 @@
 //      pos(row, k) = k * PITCH + row,  PITCH = ROWS + 16.
 //    The 16-element pad puts consecutive k-rows 32 banks (FP64) / 16 banks (FP32) apart,
 //    so the 16 rows x 2 (FP64) or 4 (FP32) k values one MFMA fragment read touches are
-//    on distinct banks.
+//    on distinct banks. Where a 16-byte instruction (1024 bytes) spans KPI > 1 k-rows (FP32
+//    up to 128 rows, FP64 64 rows) those are contiguous, the padding stands between groups of
+//    KPI, and within a group block i of 16 rows of k-row x sits at block i ^ x, which does for
+//    the banks what the pad does elsewhere:
+//      pos(row, k) = (k / KPI) * GPITCH + (k % KPI) * ROWS + (row ^ 16 * (k % KPI)).
 //  - KROW (source contiguous along k): each tile row holds its BK elements as 16-byte
 //    chunks (CE = 16 bytes / element elements each), the chunk index XOR-swizzled by
 //    SW(row) = (row / RB) % NC, RB = rows per 64 banks, NC = chunks per row:
@@ -41,18 +45,22 @@ struct SlabLayout {
     static constexpr int CE    = 4 / EW;                 // elements per 16-byte chunk
     static constexpr int NC    = BK / CE;                // chunks per KROW row
     static constexpr int RB    = 64 / (BK * EW);         // KROW rows per 64 banks
+    // KMAJOR: k-rows per instruction, when one spans several whole ones
+    static constexpr int KPI   = !KROW && 64 * VW > ROWS * EW && (64 * VW) % (ROWS * EW) == 0 ? 64 * VW / (ROWS * EW) : 1;
     static constexpr int PITCH = ROWS + 16;              // KMAJOR k-row pitch (elements)
-    static constexpr int SIZE  = KROW ? ROWS * BK : BK * PITCH; // elements per buffer
+    static constexpr int GPITCH = KPI * ROWS + (KPI == 2 && EW == 1 ? 32 : 16); // KMAJOR group pitch, KPI > 1
+    static constexpr int SIZE  = KROW ? ROWS * BK : KPI > 1 ? BK / KPI * GPITCH : BK * PITCH; // elements per buffer
     static constexpr int SLAB_DW = ROWS * BK * EW;       // dwords moved per slab
     static constexpr int INS   = SLAB_DW / (64 * VW);    // wave instructions per slab
     static constexpr int INS_PER_WAVE = INS / 4;
     // KMAJOR: instructions per k-row (a wide instruction must not span two padded k-rows)
-    static constexpr int IPR = KROW ? 1 : (ROWS * EW) / (64 * VW);
+    static constexpr int IPR = KROW || KPI > 1 ? 1 : (ROWS * EW) / (64 * VW);
     static constexpr bool VALID = IPR >= 1 && INS % 4 == 0 && BK % CE == 0 && RB >= 1 && NC >= 1;
 
     static __host__ __device__ constexpr int sw(int row) { return (row / RB) % NC; }
     static __host__ __device__ constexpr int pos(int row, int k) {
-        return KROW ? row * BK + ((k / CE) ^ sw(row)) * CE + k % CE : k * PITCH + row;
+        if (KROW) return row * BK + ((k / CE) ^ sw(row)) * CE + k % CE;
+        return KPI > 1 ? (k / KPI) * GPITCH + (k % KPI) * ROWS + (row ^ (16 * (k % KPI))) : k * PITCH + row;
     }
     // KMAJOR: instruction n = w + 4x (wave w, x-th instruction of the wave) covers part
     // n % IPR of k-row n / IPR. Written per case so that the compiler sees that a lane
@@ -65,7 +73,9 @@ struct SlabLayout {
     }
     // First LDS dword written by instruction (w, x).
     static __host__ __device__ constexpr int ins_base_dw(int w, int x) {
-        return KROW ? (w + 4 * x) * 64 * VW : group_of(w, x) * PITCH * EW + part_of(w, x) * 64 * VW;
+        return KROW      ? (w + 4 * x) * 64 * VW
+               : KPI > 1 ? (w + 4 * x) * GPITCH * EW
+                         : group_of(w, x) * PITCH * EW + part_of(w, x) * 64 * VW;
     }
     // Element (row, k) and dword half h that lane l of instruction (w, x) copies (for WIDE,
     // the first element of its 16-byte chunk; the chunk runs along rows for KMAJOR, along
@@ -78,6 +88,11 @@ struct SlabLayout {
             int const cs = (e % BK) / CE; // chunk slot in the row
             k            = (cs ^ sw(row)) * CE + e % CE;
             h            = d % EW;
+        } else if (KPI > 1) {
+            int const e = l * VW / EW; // element inside the group
+            k           = (w + 4 * x) * KPI + e / ROWS;
+            row         = (e % ROWS) ^ (16 * (e / ROWS));
+            h           = 0;
         } else {
             int const o = part_of(w, x) * 64 * VW + l * VW; // dword inside the k-row
             row         = o / EW;
@@ -157,6 +172,14 @@ __device__ __forceinline__ void mfma_slab_lds(T const *__restrict__ As, T const 
     }
 }
 
+// Whether a tile of `rows` rows has a k-major layout for 16-byte DMA: an instruction covers part
+// of a k-row or a whole number of them.
+template <typename T>
+constexpr bool kmajor_wide(int rows) {
+    int const dw = rows * int(sizeof(T)) / 4;
+    return dw >= 256 || 256 % dw == 0;
+}
+
 // Staging choice for one operand (host side): KROW layout when the source is contiguous
 // along k, 16-byte DMA when every chunk is contiguous, 16-byte aligned and entirely
 // inside or outside the problem.
@@ -168,15 +191,14 @@ struct OperandStaging {
 template <typename T>
 inline OperandStaging choose_staging(int rows_tile, int64_t s_row, int64_t s_k, int64_t s_batch, int64_t batch,
                                      int64_t rows, int64_t K, void const *ptr) {
-    constexpr int EW = int(sizeof(T)) / 4;
-    constexpr int KG = 4 / EW;
+    constexpr int KG = 16 / int(sizeof(T));
     auto mag         = [](int64_t x) { return x < 0 ? -x : x; };
     OperandStaging st{};
     bool const row_fast = s_row == 1 || (s_k != 1 && mag(s_row) <= mag(s_k));
     st.krow             = !row_fast;
     bool const aligned  = reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && (batch <= 1 || s_batch % KG == 0);
     if (!st.krow)
-        st.wide = aligned && s_row == 1 && s_k % KG == 0 && rows % KG == 0 && rows_tile * EW >= 256;
+        st.wide = aligned && s_row == 1 && s_k % KG == 0 && rows % KG == 0 && kmajor_wide<T>(rows_tile);
     else
         st.wide = aligned && s_k == 1 && s_row % KG == 0 && K % KG == 0;
     return st;
