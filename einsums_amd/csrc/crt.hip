@@ -13,10 +13,11 @@
 //      launches): R_l = (a_l b_l) mod m_l in [0, m_l), stored as bytes.
 //   4. Reconstruction: S = sum_l R_l W_l with W_l the CRT basis of M = prod m_l, and
 //      C' = S - M rint(S / M), the representative in (-M/2, M/2). kb is the largest value
-//      with 4 K 2^(2 kb) <= M, so |A'B'| <= M/4 and C' = A'B' exactly. W_l and M are kept
-//      as four 32-bit limbs (M < 2^128 for 16 moduli), so every limb sum of S and every limb
-//      of S - qM is an exact FP64 integer below 2^45; the limbs of C' are then added as a
-//      double-double (error-free two-sums), which rounds C' once even where its limbs cancel.
+//      with 4 K 2^(2 kb) <= M, so |A'B'| <= M/4 and C' = A'B' exactly. W_l and M are kept in
+//      limbs of 40 bits (three, up to 15 moduli) or 32 bits (four, 16 moduli), so every limb
+//      sum of S and every limb of S - qM is an exact FP64 integer; the limbs of C' are then
+//      added as a double-double (error-free two-sums), which rounds C' once even where its
+//      limbs cancel.
 //      C = alpha C' 2^(e_i + f_j - 2 kb) + beta C.
 //
 // Every product of A' and B' is formed exactly, so the only error is the rounding of A
@@ -24,8 +25,12 @@
 // 13 moduli give kb = 44 at K = 2304 and 42 at K = 65536.
 //
 // Against the 21 products of six int8 slices, L moduli take L int8 GEMMs, each with one
-// int32 accumulator per output: the GEMM here can use 256 x 256 tiles and a four-deep
-// LDS ring, where six slices leave room for 128 x 64 tiles and two stages.
+// int32 accumulator per output, where six slices leave room for 128 x 64 tiles only.
+//
+// The residue planes are stored as the GEMM stages them: blocks of 16 rows by 64 steps, 1024
+// consecutive bytes (blocks of a row group along k), so that every DMA instruction reads eight
+// whole cache lines. Row-major planes gave it sixteen halves, and at the same bytes twice the
+// requests (4096^3, 12 moduli: 1378 -> 1259 us from this alone).
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -52,26 +57,39 @@ struct CrtMods {
     int32_t nmod;
     int32_t kbits;
     int32_t mod[CRT_MAX_MODS];
-    uint32_t magic[CRT_MAX_MODS]; // floor(2^32 / m)
-    uint32_t bias[CRT_MAX_MODS];  // m * ceil(2^30 / m): makes an int32 in [-2^30, 2^30 + 2^8) non-negative
+    int32_t c15[CRT_MAX_MODS];    // 2^15 mod m, symmetric
+    float finv[CRT_MAX_MODS];     // 1 / m
     double rinv[CRT_MAX_MODS];    // 1 / m
 };
+
+// Limbs of M and of the CRT basis: three of 40 bits up to 15 moduli (M < 2^120: a sum of 15
+// products of a residue byte and a limb stays below 2^52, an exact FP64 integer), four of 32
+// for 16.
+constexpr int crt_limbs(int nmod) { return nmod < 16 ? 3 : 4; }
+constexpr int crt_limb_bits(int limbs) { return limbs == 3 ? 40 : 32; }
 
 struct CrtBasis {
     int32_t nmod;
     int32_t shift;             // 2 kb
-    double w[CRT_MAX_MODS][4]; // W_l = w0 + w1 2^32 + w2 2^64 + w3 2^96
+    double w[CRT_MAX_MODS][4]; // W_l in limbs, lowest first
     double mlimb[4];           // M in the same limbs
     double inv_m;              // 1 / M (rounded)
 };
 
 // ------------------------------------------------------------------ residues
-// 64 x 64 tiles of X staged through LDS so that the read follows X's unit-stride axis;
-// residues written along p: out[l][r][kp]. Each thread takes four consecutive p of four rows
-// and writes one 32-bit word (four residues) per row and modulus.
-template <bool ROWS_FAST>
+// 64 x 64 tiles of X staged through LDS so that the read follows X's unit-stride axis. Each
+// thread takes four consecutive p of four rows and writes one 32-bit word (four residues) per
+// row and modulus into the blocked plane.
+// FAST (kb <= 50): with q = rint(x/m) in the low bits of x rinv + 1.5 2^52, the residue's byte
+// is the low byte of x - q m = x + q (256 - m) mod 256: one FP64 and one 24-bit operation. The
+// product with the rounded 1/m is off by less than 2^(50 - 7.6 - 53) = 2^-10.6, and x/m is at
+// least 1/(2m) >= 2^-9 from a tie (m odd; for m = 256 either tie is the same byte), so q is the
+// nearest integer. Above 50 bits the quotient may be one off and is corrected. 134 MB of
+// operand to 12 moduli: 143 -> 85 us.
+template <bool ROWS_FAST, bool FAST>
 __global__ __launch_bounds__(256) void crt_residue_kernel(SliceSrc S, int32_t const *__restrict__ e, CrtMods K,
-                                                          int8_t *__restrict__ out) {
+                                                          int8_t *__restrict__ out, int64_t plane) {
+    constexpr double ROUND = 0x1.8p52; // x + ROUND: x rounded to an integer, in the low bits
     __shared__ double tile[64][65];
     int64_t const r0 = int64_t(blockIdx.y) * 64;
     int64_t const p0 = int64_t(blockIdx.x) * 64;
@@ -104,40 +122,55 @@ __global__ __launch_bounds__(256) void crt_residue_kernel(SliceSrc S, int32_t co
         if (r >= S.rows) continue;
         int const sh = K.kbits - e[r];
         double x[4];
+        uint32_t xl[4]; // x mod 2^32
 #pragma unroll
-        for (int u = 0; u < 4; ++u) x[u] = rint(ldexp(tile[lr][p4 + u], sh)); // |x| <= 2^kb, exact
-        int8_t *__restrict__ dst = out + r * S.kp + p;
-#pragma unroll 1
-        for (int l = 0; l < K.nmod; ++l) {
-            double const m  = double(K.mod[l]);
-            double const hi = K.mod[l] == 256 ? 127.0 : 0.5 * (m - 1.0);
-            double const lo = K.mod[l] == 256 ? -128.0 : -hi;
-            uint32_t word   = 0;
+        for (int u = 0; u < 4; ++u) {
+            x[u]  = rint(ldexp(tile[lr][p4 + u], sh)); // |x| <= 2^kb, exact
+            xl[u] = FAST ? uint32_t(__double2loint(x[u] + ROUND)) : 0u;
+        }
+        int8_t *__restrict__ dst = out + (r >> 4) * 16 * S.kp + (p0 >> 6) * 1024 + (r & 15) * 64 + p4;
+        if constexpr (FAST) {
+#pragma unroll 4
+            for (int l = 0; l < K.nmod; ++l) {
+                uint32_t b[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                double v = fma(-rint(x[u] * K.rinv[l]), m, x[u]); // x - m*q: an exact small integer
-                v        = v > hi ? v - m : v;
-                v        = v < lo ? v + m : v;
-                word |= uint32_t(uint8_t(int8_t(v))) << (8 * u);
+                for (int u = 0; u < 4; ++u)
+                    b[u] = __umul24(uint32_t(__double2loint(fma(x[u], K.rinv[l], ROUND))), uint32_t(256 - K.mod[l])) + xl[u];
+                uint32_t const lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
+                *reinterpret_cast<uint32_t *>(dst + int64_t(l) * plane) = lo | hi;
             }
-            *reinterpret_cast<uint32_t *>(dst + int64_t(l) * S.rows * S.kp) = word;
+        } else {
+#pragma unroll 1
+            for (int l = 0; l < K.nmod; ++l) {
+                double const m  = double(K.mod[l]);
+                double const hi = K.mod[l] == 256 ? 127.0 : 0.5 * (m - 1.0);
+                double const lo = K.mod[l] == 256 ? -128.0 : -hi;
+                uint32_t word   = 0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    double v = fma(-rint(x[u] * K.rinv[l]), m, x[u]); // x - m*q: an exact small integer
+                    v        = v > hi ? v - m : v;
+                    v        = v < lo ? v + m : v;
+                    word |= uint32_t(uint8_t(int8_t(v))) << (8 * u);
+                }
+                *reinterpret_cast<uint32_t *>(dst + int64_t(l) * plane) = word;
+            }
         }
     }
 }
 
 // ------------------------------------------------------------- residue GEMM
-// R_l(j, i) = (sum_p a_l(i,p) b_l(j,p)) mod m_l for all moduli in one launch. Workgroup
-// tile 256 x 256 (i x j), eight waves (two per SIMD) of 128 x 64: 8 x 4 blocks of the
-// 16 x 16 x 64 int8 MFMA, 128 int32 accumulators per lane. Operand stages of 64
-// contraction steps go global -> LDS by DMA through a ring of four buffers.
-constexpr int CG_TILE = 256, CG_KS = 64, CG_NBUF = 4, CG_WAVES = 8;
-constexpr int CG_SLOTS = CG_TILE * 4;                 // 16-byte chunks per operand stage
-constexpr int CG_DMA   = CG_SLOTS / 64 / CG_WAVES;    // DMA instructions per operand, wave and stage
+// R_l(j, i) = (sum_p a_l(i,p) b_l(j,p)) mod m_l for all moduli in one launch, as a byte in
+// [0, m_l].
+constexpr int CG_TI = 256, CG_TJ = 128, CG_KS = 64, CG_NBUF = 3, CG_WAVES = 4;
+constexpr int CG_SA = CG_TI * 4, CG_SB = CG_TJ * 4;   // 16-byte chunks per operand stage
+constexpr int CG_DA = CG_SA / 64 / CG_WAVES, CG_DB = CG_SB / 64 / CG_WAVES; // DMA instructions per wave and stage
 
 struct CrtGemm {
     int64_t m, n, kp;         // rows of a (i), rows of b (j, this panel), padded contraction length
     int64_t k0, kc;           // contraction steps [k0, k0 + kc) of this launch (multiples of 64)
     int32_t accumulate;       // add to the stored residues instead of overwriting them
+    uint32_t items;           // (modulus, tile) pairs
     int64_t a_plane, b_plane; // elements between the moduli of the residue operands
     int8_t const *A;
     int8_t const *B;
@@ -147,71 +180,54 @@ struct CrtGemm {
     CrtMods K;
 };
 
-// chunk c of row `row` sits at slot row*4 + (c ^ ((row >> 2) & 3)): the 16 rows of one
-// fragment read fall on distinct 16-byte bank groups
-__device__ __forceinline__ int cg_slot(int row, int c) { return row * 4 + (c ^ ((row >> 2) & 3)); }
+// 16-byte chunk c of row `row` of an operand sits at slot row*4 + (c ^ f(row)); f puts the 16
+// rows of one fragment read (see the kernel) on distinct 16-byte bank groups.
+template <bool A>
+__device__ __forceinline__ int cg_swz(int row) { return A ? (row >> 5) & 3 : (row >> 2) & 3; }
 
-// One operand stage: lane l of instruction n (n = wave, wave + 8) fills slot 64n + l.
-__device__ __forceinline__ void cg_dma(int8_t const *__restrict__ X, int64_t rows, int64_t kp, int64_t row0, int64_t k0,
-                                       int8_t *lds, int wave, int lane) {
+// Workgroup barrier that no memory access of the code is moved across.
+__device__ __forceinline__ void cg_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// One operand stage: lane l of instruction n = wave + 4x fills slot 64n + l, i.e. chunk l % 4
+// (swizzled) of row 16n + l / 4, out of block n of the stage. `tile` is the tile's first block,
+// `off` the lane's offset for x = 0; the swizzle of A moves the chunk by two for odd x. Rows
+// beyond the operand are whatever follows in the workspace: they only reach outputs that are
+// not stored, or lie in the padding of R.
+template <bool A, int N>
+__device__ __forceinline__ void cg_dma(int8_t const *__restrict__ tile, int64_t kp, int64_t off, int8_t *lds, int wave) {
 #pragma unroll
-    for (int x = 0; x < CG_DMA; ++x) {
-        int const n     = wave + CG_WAVES * x;
-        int const sl    = n * 64 + lane;
-        int const row   = sl >> 2;
-        int const c     = (sl & 3) ^ ((row >> 2) & 3);
-        int64_t const g = row0 + row;
-        void const *src = g < rows ? static_cast<void const *>(X + g * kp + k0 + 16 * c)
-                                   : static_cast<void const *>(ein_zero_page);
-        __builtin_amdgcn_global_load_lds(src, EIN_LDS_PTR(lds + n * 64 * 16), 16, 0, 0);
+    for (int x = 0; x < N; ++x) {
+        int8_t const *src = tile + 64 * x * kp + (A && (x & 1) ? off ^ 32 : off);
+        __builtin_amdgcn_global_load_lds(src, EIN_LDS_PTR(lds + (wave + CG_WAVES * x) * 64 * 16), 16, 0, 0);
     }
 }
 
-// x mod m in [0, m) for x in [-2^30, 2^30 + 2^8): Barrett with floor(2^32/m), which is low
-// by at most two.
-__device__ __forceinline__ uint32_t cg_mod(int32_t x, uint32_t m, uint32_t magic, uint32_t bias) {
-    uint32_t const u = uint32_t(x) + bias;
-    uint32_t r       = u - __umulhi(u, magic) * m;
-    r                = r >= m ? r - m : r;
-    r                = r >= m ? r - m : r;
-    return r;
-}
-
-__device__ __forceinline__ void cg_load_b(int8_t const *__restrict__ stage, v4i (&bf)[4], int wn, int r, int q) {
-    v4i const *Bs = reinterpret_cast<v4i const *>(stage) + CG_SLOTS;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) bf[b] = Bs[cg_slot(wn * 64 + b * 16 + r, q)];
-}
-
-__device__ __forceinline__ v4i cg_load_a(int8_t const *__restrict__ stage, int a, int wm, int r, int q) {
-    return reinterpret_cast<v4i const *>(stage)[cg_slot(wm * 128 + a * 16 + r, q)];
-}
-
-// Waits until at most `pending` later stages of this wave's DMA are outstanding, then for
-// the whole workgroup.
-__device__ __forceinline__ void cg_wait(int pending) {
-    static_assert(2 * CG_DMA == 4, "vmcnt counts below assume 4 DMA instructions per wave and stage");
-    if (pending >= 3)
-        asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-    else if (pending == 2)
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else if (pending == 1)
-        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-}
-
-// Residue GEMM of one (modulus, tile) per workgroup. Stage s sits in LDS buffer s % 4, and
-// four stages are in flight when the loop starts. Within stage s each wave runs its eight
-// row blocks of a against the four b fragments held in registers, reading the next a
-// fragment ahead of each block's MFMAs. Halfway through, it waits for stage s+1 and reads
-// that stage's b fragments into the second register set; after the last block a barrier
-// (every wave has read stage s) frees buffer s % 4 for the DMA of stage s+4.
+// Persistent: two workgroups per CU, each walking every grid-th (modulus, 256 x 128 tile), four
+// waves of 128 x 64, 8 x 4 blocks of the 16 x 16 x 64 int8 MFMA. 64-step operand stages go
+// global -> LDS by DMA through a ring of three buffers. While a stage's 32 MFMAs run from
+// registers, the next stage's fragments are read and the DMA of the one three ahead is issued
+// into the buffer just read; one barrier a stage. The next item's first stages are in flight
+// during the epilogue.
+// At k = 1024 a tile has 16 stages, about as long as its epilogue (the reduction of 128
+// accumulators a lane), so what matters is that the other workgroup's MFMAs run meanwhile: one
+// 256 x 256 tile per CU in lockstep took 5214 us for 16384^2 x 1024, 12 moduli (MFMA busy 26%
+// of 12.0M cycles at 2.19 GHz), this 4108 (42% of 7.5M cycles at 1.79 GHz: it is now the power
+// limit that sets the clock). 4096^3 in all 1339 -> 1057 us, 2304^2 x 65536 9.32 -> 7.53 ms.
+//
+// Row 16a + r of a wave's A fragment a is row (r/4)*32 + 4a + r%4 of its 128: with that order
+// a lane's results of one column are 32 consecutive bytes of R, two 16-byte stores.
+// The reduction mod m: x = 2^15 hi + lo -> hi (2^15 mod m) + lo, below 2^23 in magnitude and
+// exact in 24-bit integer arithmetic and FP32; then y - m floor(y / m), whose floor is right or,
+// at a multiple of m, one low, which stores m for 0: the same residue, and m <= 255 (for 256
+// the division is exact) still fits the byte.
 // The contraction is at most CRT_FOLD_STAGES stages (|int32 sum| <= 2^30); longer ones run
 // as several launches with `accumulate` set, each adding its residues to the stored ones.
-__global__ __launch_bounds__(64 * CG_WAVES, 1) void crt_gemm_kernel(CrtGemm P) {
-    __shared__ __attribute__((aligned(16))) int8_t lds[CG_NBUF * 2 * CG_SLOTS * 16];
+__global__ __launch_bounds__(64 * CG_WAVES, 2) void crt_gemm_kernel(CrtGemm P) {
+    __shared__ __attribute__((aligned(16))) int8_t lds[CG_NBUF * (CG_SA + CG_SB) * 16];
 
     int const tid  = threadIdx.x;
     int const lane = tid & 63;
@@ -220,91 +236,145 @@ __global__ __launch_bounds__(64 * CG_WAVES, 1) void crt_gemm_kernel(CrtGemm P) {
     int const wn   = wave >> 1;
     int const r    = lane & 15;
     int const q    = lane >> 4;
+    // fragment slots of this lane: A row (r/4)*32 + 4a + r%4 of the wave's 128, B row 16b + r
+    int const a_row = wm * 128 + (r >> 2) * 32 + (r & 3);
+    int const a_sl  = a_row * 4 + (q ^ cg_swz<true>(a_row)); // + 16 a: the swizzle depends on r/4 only
+    int const b_row = wn * 64 + r;
+    int const b_sl  = CG_SA + b_row * 4 + (q ^ cg_swz<false>(b_row)); // + 64 b
 
-    uint32_t const ntiles  = P.tiles_m * P.tiles_n;
-    uint32_t const logical = xcd_remap(blockIdx.x, gridDim.x);
-    uint32_t const l       = logical / ntiles;
-    uint32_t const tile    = logical - l * ntiles;
-    uint32_t tm, tn;
-    tile_coords(tile, P.tiles_m, P.tiles_n, tm, tn);
-    int64_t const i0 = int64_t(tm) * CG_TILE;
-    int64_t const j0 = int64_t(tn) * CG_TILE;
-    int8_t const *__restrict__ Ag = P.A + int64_t(l) * P.a_plane + P.k0;
-    int8_t const *__restrict__ Bg = P.B + int64_t(l) * P.b_plane + P.k0;
-
-    v4i acc[8][4];
-#pragma unroll
-    for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = v4i{0, 0, 0, 0};
-
-    auto buf = [&](int64_t s) { return lds + (s & (CG_NBUF - 1)) * (2 * CG_SLOTS * 16); };
-    auto dma = [&](int64_t s) {
-        int8_t *dst = buf(s);
-        cg_dma(Ag, P.m, P.kp, i0, s * CG_KS, dst, wave, lane);
-        cg_dma(Bg, P.n, P.kp, j0, s * CG_KS, dst + CG_SLOTS * 16, wave, lane);
+    uint32_t const ntiles = P.tiles_m * P.tiles_n;
+    int64_t const nst     = P.kc / CG_KS;
+    auto buf = [&](int z) { return lds + z * ((CG_SA + CG_SB) * 16); };
+    struct Item {
+        int8_t const *A, *B;
+        int64_t i0, j0;
+        uint32_t l;
     };
-    int64_t const nst = P.kc / CG_KS;
-    for (int64_t s = 0; s < nst && s < CG_NBUF; ++s) dma(s);
-    cg_wait(int(nst - 1 < 3 ? nst - 1 : 3));
-    v4i b0[4], b1[4];
-    cg_load_b(buf(0), b0, wn, r, q);
-    v4i an = cg_load_a(buf(0), 0, wm, r, q);
+    auto item_of = [&](uint32_t it) {
+        Item x;
+        x.l                 = it / ntiles;
+        uint32_t const tile = it - x.l * ntiles;
+        uint32_t tm, tn;
+        tile_coords(tile, P.tiles_m, P.tiles_n, tm, tn);
+        x.i0 = int64_t(tm) * CG_TI;
+        x.j0 = int64_t(tn) * CG_TJ;
+        x.A  = P.A + int64_t(x.l) * P.a_plane + P.k0 * 16 + x.i0 * P.kp;
+        x.B  = P.B + int64_t(x.l) * P.b_plane + P.k0 * 16 + x.j0 * P.kp;
+        return x;
+    };
+    int const d_row     = wave * 16 + (lane >> 2);
+    int64_t const a_off = wave * 16 * P.kp + (lane >> 2) * 64 + 16 * ((lane & 3) ^ cg_swz<true>(d_row));
+    int64_t const b_off = wave * 16 * P.kp + (lane >> 2) * 64 + 16 * ((lane & 3) ^ cg_swz<false>(d_row));
+    auto dma = [&](Item const &x, int64_t s, int z) {
+        int8_t *dst = buf(z);
+        cg_dma<true, CG_DA>(x.A + s * 1024, P.kp, a_off, dst, wave);
+        cg_dma<false, CG_DB>(x.B + s * 1024, P.kp, b_off, dst + CG_SA * 16, wave);
+    };
+    uint32_t it = xcd_remap(blockIdx.x, gridDim.x);
+    if (it >= P.items) return;
+    Item cur = item_of(it);
+    for (int s = 0; s < CG_NBUF && s < nst; ++s) dma(cur, s, s);
 
-#define CG_STAGE(BC, BN, ST)                                                                                           \
-    do {                                                                                                               \
-        int8_t const *cur_ = buf(ST);                                                                                  \
-        bool const more_   = (ST) + 1 < nst;                                                                           \
-        _Pragma("unroll") for (int a = 0; a < 8; ++a) {                                                                \
-            v4i const af = an;                                                                                         \
-            if (a < 7)                                                                                                 \
-                an = cg_load_a(cur_, a + 1, wm, r, q);                                                                 \
-            else if (more_)                                                                                            \
-                an = cg_load_a(buf((ST) + 1), 0, wm, r, q);                                                            \
-            _Pragma("unroll") for (int b = 0; b < 4; ++b) acc[a][b] =                                                  \
-                __builtin_amdgcn_mfma_i32_16x16x64_i8(af, BC[b], acc[a][b], 0, 0, 0);                                   \
-            if (a == 3 && more_) {                                                                                     \
-                int64_t const after_ = nst - 2 - (ST); /* stages issued beyond ST+1 */                                 \
-                cg_wait(int(after_ < 2 ? after_ : 2));                                                                 \
-                cg_load_b(buf((ST) + 1), BN, wn, r, q);                                                                \
-            }                                                                                                          \
-        }                                                                                                              \
-        if ((ST) + CG_NBUF < nst) {                                                                                    \
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                          \
-            __builtin_amdgcn_s_barrier();                                                                              \
-            dma((ST) + CG_NBUF);                                                                                       \
-        }                                                                                                              \
-    } while (0)
-
-    for (int64_t st = 0; st < nst; st += 2) {
-        CG_STAGE(b0, b1, st);
-        if (st + 1 < nst) CG_STAGE(b1, b0, st + 1);
-    }
-#undef CG_STAGE
-
-    // D[4*(lane/16)+v][lane%16] of block (a, b): i = ... + 4q + v, j = ... + r
-    uint32_t const m     = uint32_t(P.K.mod[l]);
-    uint32_t const magic = P.K.magic[l];
-    uint32_t const bias  = P.K.bias[l];
-    uint8_t *__restrict__ Rl = P.R + int64_t(l) * P.r_plane;
+    for (;;) {
+        v4i acc[8][4];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        int64_t const j = j0 + wn * 64 + b * 16 + r;
-        if (j >= P.n) continue;
+        for (int a = 0; a < 8; ++a)
 #pragma unroll
-        for (int a = 0; a < 8; ++a) {
-            int64_t const i    = i0 + wm * 128 + a * 16 + 4 * q; // < ldr (padded to whole tiles)
-            uint32_t *dst      = reinterpret_cast<uint32_t *>(Rl + j * P.ldr + i);
-            uint32_t const old = P.accumulate ? *dst : 0u;
-            uint32_t word      = 0;
+            for (int b = 0; b < 4; ++b) acc[a][b] = v4i{0, 0, 0, 0};
+        v4i fa[2][8], fb[2][4];
+        auto frags = [&](int8_t const *__restrict__ st, v4i (&xa)[8], v4i (&xb)[4]) {
+            v4i const *p = reinterpret_cast<v4i const *>(st);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                uint32_t x = cg_mod(acc[a][b][v], m, magic, bias) + ((old >> (8 * v)) & 0xffu);
-                x          = x >= m ? x - m : x;
-                word |= x << (8 * v);
+            for (int a = 0; a < 8; ++a) xa[a] = p[a_sl + 16 * a];
+#pragma unroll
+            for (int b = 0; b < 4; ++b) xb[b] = p[b_sl + 64 * b];
+        };
+        // the first stage (and the last item's stores)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        cg_barrier();
+        frags(buf(0), fa[0], fb[0]);
+        int z = 0; // buffer of stage s
+        auto stage = [&](int64_t s, v4i (&xa)[8], v4i (&xb)[4], v4i (&ya)[8], v4i (&yb)[4]) {
+            int const z1 = z == CG_NBUF - 1 ? 0 : z + 1;
+            if (s + 1 < nst) {
+                // stage s+2 may stay in flight (the item's first three were waited for)
+                static_assert(CG_DA + CG_DB == 6 && CG_NBUF == 3, "the vmcnt below");
+                if (s + 2 < nst && s > 0)
+                    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+                else
+                    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                cg_barrier(); // stage s+1 is there, and every wave has read stage s
+                if (s + 3 < nst) dma(cur, s + 3, z);
+                frags(buf(z1), ya, yb);
             }
-            *dst = word;
+            z = z1;
+#pragma unroll
+            for (int a = 0; a < 8; ++a)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[a], xb[b], acc[a][b], 0, 0, 0);
+        };
+        for (int64_t s = 0; s < nst; s += 2) {
+            stage(s, fa[0], fb[0], fa[1], fb[1]);
+            if (s + 1 < nst) stage(s + 1, fa[1], fb[1], fa[0], fb[0]);
         }
+        // every wave has read its last fragments: the ring is free for the next item
+        uint32_t const nx = it + gridDim.x;
+        Item next         = cur;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        cg_barrier();
+        if (nx < P.items) {
+            next = item_of(nx);
+            for (int s = 0; s < CG_NBUF && s < nst; ++s) dma(next, s, s);
+        }
+        // D[4q+v][r] of block (a, b): i = wm*128 + 32q + 4a + v, j = wn*128 + 16b + r: a lane's
+        // 32 consecutive bytes of column j
+        float const m    = float(P.K.mod[cur.l]);
+        float const inv  = P.K.finv[cur.l];
+        int const c15    = P.K.c15[cur.l];
+        uint8_t *__restrict__ Rl = P.R + int64_t(cur.l) * P.r_plane + cur.i0 + wm * 128 + q * 32;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            int64_t const j = cur.j0 + wn * 64 + b * 16 + r;
+            if (j >= P.n) continue;
+            v4i *dst = reinterpret_cast<v4i *>(Rl + j * P.ldr);
+            v4i out[2];
+#pragma unroll
+            for (int a = 0; a < 8; ++a) {
+                uint32_t word = 0;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    int const x = acc[a][b][v];
+                    float const y = float(__mul24(x >> 15, c15) + (x & 0x7fff)); // exact: below 2^23
+                    float const t = fmaf(-floorf(y * inv), m, y);                // in [0, m]
+                    word = __builtin_amdgcn_cvt_pk_u8_f32(t, v, word);
+                }
+                out[a >> 2][a & 3] = int(word);
+            }
+            if (P.accumulate) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    v4i const old = dst[h];
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        uint32_t const o = uint32_t(old[w]), n = uint32_t(out[h][w]);
+                        uint32_t word = 0;
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            uint32_t x = ((o >> (8 * v)) & 0xffu) + ((n >> (8 * v)) & 0xffu);
+                            x = x >= uint32_t(P.K.mod[cur.l]) ? x - uint32_t(P.K.mod[cur.l]) : x;
+                            x = x >= uint32_t(P.K.mod[cur.l]) ? x - uint32_t(P.K.mod[cur.l]) : x;
+                            word |= x << (8 * v);
+                        }
+                        out[h][w] = int(word);
+                    }
+                }
+            }
+            dst[0] = out[0];
+            dst[1] = out[1];
+        }
+        if (nx >= P.items) break;
+        it  = nx;
+        cur = next;
     }
 }
 
@@ -330,47 +400,88 @@ __device__ __forceinline__ double two_sum(double a, double b, double &e) {
     return s;
 }
 
+// Bytes 0..3 of a word as doubles: the byte under the exponent of 2^52, minus 2^52 (two
+// full-rate operations, against a quarter-rate conversion).
+__device__ __forceinline__ double byte_to_double(uint32_t word, int v) {
+    return __hiloint2double(0x43300000, int((word >> (8 * v)) & 0xffu)) - 0x1p52;
+}
+
+// HBM-bound: L bytes of residues and 8 or 16 of C per element. All residue words and C are
+// requested before the arithmetic, C moves as 16-byte vectors where it can, three 40-bit limbs
+// take a quarter fewer products than four of 32 bits. 16384^2, 12 moduli, beta = 1 (7.5 GB):
+// 1935 -> 1468 us (5.1 TB/s).
+template <int NL, bool VEC>
 __global__ __launch_bounds__(256) void crt_reconstruct_kernel(CrtRec P) {
+    constexpr double B1 = NL == 3 ? 0x1p40 : 0x1p32, B2 = B1 * B1, B3 = B2 * B1;
     int64_t const words = P.ldr / 4;
     int64_t const g     = int64_t(blockIdx.x) * 256 + threadIdx.x;
     int64_t const j     = g / words;
     int64_t const i     = (g - j * words) * 4;
     if (j >= P.n || i >= P.m) return;
-    double s[4][4];
+    uint8_t const *__restrict__ src = P.R + j * P.ldr + i;
+    double *const c                 = P.C + i * P.c_sm + j * P.c_sn;
+    // all reads first
+    uint32_t word[CRT_MAX_MODS];
+#pragma unroll
+    for (int l = 0; l < CRT_MAX_MODS; ++l)
+        if (l < P.W.nmod) word[l] = *reinterpret_cast<uint32_t const *>(src + int64_t(l) * P.r_plane);
+    double old[4] = {0.0, 0.0, 0.0, 0.0};
+    bool const whole = i + 4 <= P.m;
+    if (P.beta != 0.0) {
+        if (VEC && whole) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                double2 const t = *reinterpret_cast<double2 const *>(c + 2 * h);
+                old[2 * h]      = t.x;
+                old[2 * h + 1]  = t.y;
+            }
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (i + v < P.m) old[v] = c[v * P.c_sm];
+        }
+    }
+    double s[4][NL];
 #pragma unroll
     for (int v = 0; v < 4; ++v)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) s[v][t] = 0.0;
-    uint8_t const *__restrict__ src = P.R + j * P.ldr + i;
-#pragma unroll 4
-    for (int l = 0; l < P.W.nmod; ++l) {
-        uint32_t const word = *reinterpret_cast<uint32_t const *>(src + int64_t(l) * P.r_plane);
+        for (int t = 0; t < NL; ++t) s[v][t] = 0.0;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            double const rv = double((word >> (8 * v)) & 0xffu);
+    for (int l = 0; l < CRT_MAX_MODS; ++l)
+        if (l < P.W.nmod) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) s[v][t] = fma(rv, P.W.w[l][t], s[v][t]); // exact: < 2^44
+            for (int v = 0; v < 4; ++v) {
+                double const rv = byte_to_double(word[l], v);
+#pragma unroll
+                for (int t = 0; t < NL; ++t) s[v][t] = fma(rv, P.W.w[l][t], s[v][t]); // exact
+            }
         }
-    }
     int const eb = P.eb[j];
+    double val[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        int64_t const ii = i + v;
-        if (ii >= P.m) break;
-        double const approx = fma(s[v][3], 0x1p96, fma(s[v][2], 0x1p64, fma(s[v][1], 0x1p32, s[v][0])));
-        double const qm     = rint(approx * P.W.inv_m); // S / M rounded: |C'| <= M/4 leaves margin
-        double lim[4];
+        double approx = fma(s[v][2], B2, fma(s[v][1], B1, s[v][0]));
+        if constexpr (NL == 4) approx = fma(s[v][NL - 1], B3, approx);
+        double const qm = rint(approx * P.W.inv_m); // S / M rounded: |C'| <= M/4 leaves margin
+        double lim[NL];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) lim[t] = fma(-qm, P.W.mlimb[t], s[v][t]); // exact limbs of S - qM
-        double e0, e1, e2;
-        double h = two_sum(lim[1] * 0x1p32, lim[0], e0);
-        h        = two_sum(lim[2] * 0x1p64, h, e1);
-        h        = two_sum(lim[3] * 0x1p96, h, e2);
+        for (int t = 0; t < NL; ++t) lim[t] = fma(-qm, P.W.mlimb[t], s[v][t]); // exact limbs of S - qM
+        double e0, e1, e2 = 0.0;
+        double h = two_sum(lim[1] * B1, lim[0], e0);
+        h        = two_sum(lim[2] * B2, h, e1);
+        if constexpr (NL == 4) h = two_sum(lim[NL - 1] * B3, h, e2);
         double const cp = h + ((e0 + e1) + e2);
-        double *c       = P.C + ii * P.c_sm + j * P.c_sn;
-        double val      = P.alpha * ldexp(cp, P.ea[ii] + eb - P.W.shift);
-        if (P.beta != 0.0) val = fma(P.beta, *c, val);
-        *c = val;
+        int const e     = i + v < P.m ? P.ea[i + v] : 0;
+        val[v]          = P.alpha * ldexp(cp, e + eb - P.W.shift);
+        if (P.beta != 0.0) val[v] = fma(P.beta, old[v], val[v]);
+    }
+    if (VEC && whole) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) *reinterpret_cast<double2 *>(c + 2 * h) = double2{val[2 * h], val[2 * h + 1]};
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (i + v < P.m) c[v * P.c_sm] = val[v];
     }
 }
 
@@ -400,14 +511,16 @@ void crt_constants(int nmod, int kbits, CrtMods &K, CrtBasis &W) {
     W.shift = 2 * kbits;
     u128 M  = 1;
     for (int l = 0; l < nmod; ++l) M *= u128(CRT_MODS[l]);
-    auto limbs = [](u128 x, double *out) {
-        for (int t = 0; t < 4; ++t) out[t] = double(uint64_t(x >> (32 * t)) & 0xffffffffull);
+    int const nl = crt_limbs(nmod), bits = crt_limb_bits(nl);
+    auto limbs = [&](u128 x, double *out) {
+        for (int t = 0; t < nl; ++t) out[t] = double(uint64_t(x >> (bits * t)) & ((uint64_t(1) << bits) - 1));
     };
     for (int l = 0; l < nmod; ++l) {
         uint32_t const m = uint32_t(CRT_MODS[l]);
         K.mod[l]         = int32_t(m);
-        K.magic[l]       = uint32_t((uint64_t(1) << 32) / m);
-        K.bias[l]        = uint32_t(((uint64_t(1) << 30) + m - 1) / m * m);
+        int32_t const c  = int32_t((1u << 15) % m);
+        K.c15[l]         = 2 * c > int32_t(m) ? c - int32_t(m) : c;
+        K.finv[l]        = 1.0f / float(m);
         K.rinv[l]        = 1.0 / double(m);
         u128 const Mi    = M / m;
         // inverse of Mi mod m by search (m <= 256)
@@ -424,15 +537,16 @@ void crt_constants(int nmod, int kbits, CrtMods &K, CrtBasis &W) {
     W.inv_m = 1.0 / (double(uint64_t(M >> 64)) * 0x1p64 + double(uint64_t(M)));
 }
 
-int crt_residues(SliceSrc const &S, CrtMods const &K, int32_t *e, int8_t *out, double *scratch, hipStream_t stream) {
+int crt_residues(SliceSrc const &S, CrtMods const &K, int32_t *e, int8_t *out, int64_t plane, double *scratch,
+                 hipStream_t stream) {
     bool const rows_fast = S.s_row == 1 || (S.s_k != 1 && std::llabs(S.s_row) < std::llabs(S.s_k));
     EIN_TRY(row_exponents(S, e, false, scratch, stream));
     dim3 grid{uint32_t(ceil_div(S.kp, 64)), uint32_t(ceil_div(S.rows, 64))};
     if (grid.y > 65535) return fail(EIN_ERROR_UNSUPPORTED, "split gemm: more than 4M rows");
-    if (rows_fast)
-        crt_residue_kernel<true><<<grid, 256, 0, stream>>>(S, e, K, out);
-    else
-        crt_residue_kernel<false><<<grid, 256, 0, stream>>>(S, e, K, out);
+    bool const fast   = K.kbits <= 50;
+    auto const kernel = rows_fast ? (fast ? crt_residue_kernel<true, true> : crt_residue_kernel<true, false>)
+                                  : (fast ? crt_residue_kernel<false, true> : crt_residue_kernel<false, false>);
+    kernel<<<grid, 256, 0, stream>>>(S, e, K, out, plane);
     EIN_LAUNCH_CHECK();
     return EIN_SUCCESS;
 }
@@ -490,23 +604,24 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
     CrtBasis W;
     crt_constants(nmod, kbits, K, W);
 
-    uint32_t const tiles_m = uint32_t(ceil_div(P.m, CG_TILE));
-    int64_t const ldr      = int64_t(tiles_m) * CG_TILE;
+    uint32_t const tiles_m = uint32_t(ceil_div(P.m, CG_TI));
+    int64_t const ldr      = int64_t(tiles_m) * CG_TI;
     // column panels of whole 256-column tiles whose residue planes take at most
     // CRT_PANEL_BYTES; with more than one panel, two plane buffers of half that so the
     // reconstruction of panel p (HBM-bound) runs on a side stream while the residue GEMM of
     // panel p+1 (MFMA-bound) runs on the caller's stream
     auto panel_cols = [&](size_t budget) {
-        int64_t c = int64_t(budget / (size_t(nmod) * size_t(ldr))) / CG_TILE * CG_TILE;
-        return std::max<int64_t>(CG_TILE, std::min<int64_t>(c, ceil_div(P.n, CG_TILE) * CG_TILE));
+        int64_t c = int64_t(budget / (size_t(nmod) * size_t(ldr))) / CG_TI * CG_TI;
+        return std::max<int64_t>(CG_TI, std::min<int64_t>(c, ceil_div(P.n, CG_TI) * CG_TI));
     };
     int64_t pn      = panel_cols(CRT_PANEL_BYTES);
     bool const fork = pn < P.n && !stream_capturing(stream);
     if (fork) pn = panel_cols(CRT_PANEL_BYTES / 2);
     int const nbuf = fork ? 2 : 1;
 
-    size_t const a_bytes = size_t(nmod) * size_t(P.m) * size_t(kp);
-    size_t const b_bytes = size_t(nmod) * size_t(P.n) * size_t(kp);
+    int64_t const a_plane = ceil_div(P.m, 16) * 16 * kp, b_plane = ceil_div(P.n, 16) * 16 * kp;
+    size_t const a_bytes = size_t(nmod) * size_t(a_plane);
+    size_t const b_bytes = size_t(nmod) * size_t(b_plane);
     size_t const r_bytes = size_t(nmod) * size_t(pn) * size_t(ldr);
     auto up              = [](size_t x) { return (x + 255) / 256 * 256; };
     size_t const b_off   = up(a_bytes);
@@ -514,7 +629,9 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
     size_t const ea_off  = r_off + size_t(nbuf) * up(r_bytes);
     size_t const eb_off  = ea_off + up(size_t(P.m) * 4);
     size_t const x_off   = eb_off + up(size_t(P.n) * 4);
-    size_t const total   = x_off + row_exp_scratch(std::max(P.m, P.n)) * sizeof(double);
+    // the GEMM's tiles read up to CG_TI rows past the last plane of an operand
+    size_t const total   = std::max(x_off + row_exp_scratch(std::max(P.m, P.n)) * sizeof(double),
+                                    r_off + size_t(CG_TI) * size_t(kp));
     void *ws             = nullptr;
     EIN_TRY(workspace(stream, total, &ws));
     char *base      = static_cast<char *>(ws);
@@ -527,8 +644,8 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
 
     SliceSrc SA{P.m, P.k, kp, P.A, P.a_sm, P.a_sk};
     SliceSrc SB{P.n, P.k, kp, P.B, P.b_sn, P.b_sk};
-    EIN_TRY(crt_residues(SA, K, ea, As, scratch, stream));
-    EIN_TRY(crt_residues(SB, K, eb, Bs, scratch, stream));
+    EIN_TRY(crt_residues(SA, K, ea, As, a_plane, scratch, stream));
+    EIN_TRY(crt_residues(SB, K, eb, Bs, b_plane, scratch, stream));
 
     CrtSide side;
     if (fork) EIN_TRY(crt_side(side));
@@ -543,15 +660,15 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
             G.m       = P.m;
             G.n       = nj;
             G.kp      = kp;
-            G.a_plane = P.m * kp;
-            G.b_plane = P.n * kp;
+            G.a_plane = a_plane;
+            G.b_plane = b_plane;
             G.A       = As;
             G.B       = Bs + j0 * kp;
             G.R       = Rb;
             G.ldr     = ldr;
             G.r_plane = nj * ldr;
             G.tiles_m = tiles_m;
-            G.tiles_n = uint32_t(ceil_div(nj, CG_TILE));
+            G.tiles_n = uint32_t(ceil_div(nj, CG_TJ));
             G.K       = K;
             uint64_t const grid = uint64_t(G.tiles_m) * G.tiles_n * uint64_t(nmod);
             if (grid > 0x7fffffffu) return fail(EIN_ERROR_UNSUPPORTED, "split gemm: tile grid too large");
@@ -559,7 +676,9 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
                 G.k0         = k0;
                 G.kc         = std::min<int64_t>(int64_t(CRT_FOLD_STAGES) * CG_KS, kp - k0);
                 G.accumulate = k0 > 0;
-                crt_gemm_kernel<<<uint32_t(grid), 64 * CG_WAVES, 0, stream>>>(G);
+                G.items = uint32_t(grid);
+                crt_gemm_kernel<<<uint32_t(std::min<uint64_t>(grid, 2 * uint64_t(num_cus()))), 64 * CG_WAVES, 0, stream>>>(
+                    G);
                 EIN_LAUNCH_CHECK();
             }
 
@@ -585,7 +704,10 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
             Q.W       = W;
             int64_t const threads = nj * (ldr / 4);
             if (ceil_div(threads, 256) > 0x7fffffff) return fail(EIN_ERROR_UNSUPPORTED, "split gemm: panel too large");
-            crt_reconstruct_kernel<<<uint32_t(ceil_div(threads, 256)), 256, 0, rs>>>(Q);
+            bool const vec = Q.c_sm == 1 && Q.c_sn % 2 == 0 && reinterpret_cast<uintptr_t>(Q.C) % 16 == 0;
+            auto const rec = crt_limbs(nmod) == 3 ? (vec ? crt_reconstruct_kernel<3, true> : crt_reconstruct_kernel<3, false>)
+                                                  : (vec ? crt_reconstruct_kernel<4, true> : crt_reconstruct_kernel<4, false>);
+            rec<<<uint32_t(ceil_div(threads, 256)), 256, 0, rs>>>(Q);
             if (fork) {
                 last = b;
                 EIN_HIP_CHECK(hipEventRecord(side.recon_done[b], side.aux));
