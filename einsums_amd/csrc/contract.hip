@@ -22,6 +22,7 @@
 #include "contract.hpp"
 #include "einsum.hpp"
 #include "tile_engine.hpp"
+#include "wave_tile.hpp"
 
 namespace ein {
 
@@ -768,6 +769,71 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
 
 } // namespace
 
+namespace {
+
+// One item: its problem with the index groups that its tables are built from.
+template <typename T>
+struct BuiltItem {
+    WaveItem<T> w;
+    IndexGroup gm, gn, gk, gb; // (A, C), (B, C), (A, B) and (A, B, C) strides
+    int64_t batch;
+};
+
+// The wave kernel's problem of C[b,i,j] = alpha sum_p A[b,i,p] B[b,p,j] + beta C[b,i,j], the
+// digits of each group as order_and_fold takes them.
+template <typename T>
+int build_wave(std::vector<Digit> vb, std::vector<Digit> vm, std::vector<Digit> vn, std::vector<Digit> vk, T const *pa,
+               T const *pb, T *c, T alpha, T beta, BuiltItem<T> &out) {
+    // the lanes of a wave run along i when C is read and written: the side that holds C's
+    // unit stride becomes A
+    auto unit_in_c = [](std::vector<Digit> const &v) {
+        for (auto const &d : v)
+            if (std::llabs(d.s[1]) == 1) return true;
+        return false;
+    };
+    bool const swap = unit_in_c(vn) && !unit_in_c(vm);
+    if (swap) {
+        std::swap(vm, vn);
+        std::swap(pa, pb);
+        for (auto &d : vk) std::swap(d.s[0], d.s[1]);
+        for (auto &d : vb) std::swap(d.s[0], d.s[1]);
+    }
+    auto gm = order_and_fold(vm, 2, 0, 1);
+    auto gn = order_and_fold(vn, 2, 0, 1);
+    bool const a_i_fast = !gm.empty() && std::llabs(gm.back().s[0]) == 1;
+    auto gk = a_i_fast ? order_and_fold(vk, 2, 1, 0) : order_and_fold(vk, 2, 0, 1);
+    auto gbv = order_and_fold(vb, 3, 2, 0);
+    EIN_TRY(fill_group(out.gm, gm, 2));
+    EIN_TRY(fill_group(out.gn, gn, 2));
+    EIN_TRY(fill_group(out.gk, gk, 2));
+    EIN_TRY(fill_group(out.gb, gbv, 3));
+    out.batch       = total_of(vb);
+    WaveItem<T> &w  = out.w;
+    w        = WaveItem<T>{};
+    w.A      = pa;
+    w.B      = pb;
+    w.C      = c;
+    w.alpha  = alpha;
+    w.beta   = beta;
+    w.m      = int32_t(total_of(vm));
+    w.n      = int32_t(total_of(vn));
+    w.k      = int32_t(total_of(vk));
+    // one digit: affine over all of k. Otherwise affine within 16 steps where the innermost
+    // digit's extent is a multiple of 16 (chunks start at multiples of 16)
+    w.k_mode = gk.size() <= 1 ? 2 : gk.back().e % 16 == 0 ? 1 : 0;
+    w.kA_in  = gk.empty() ? 0 : gk.back().s[0];
+    w.kB_in  = gk.empty() ? 0 : gk.back().s[1];
+    w.m_lin  = gm.size() <= 1;
+    w.n_lin  = gn.size() <= 1;
+    w.sA     = gm.empty() ? 0 : gm.back().s[0];
+    w.sC     = gm.empty() ? 0 : gm.back().s[1];
+    w.tB     = gn.empty() ? 0 : gn.back().s[0];
+    w.tC     = gn.empty() ? 0 : gn.back().s[1];
+    return EIN_SUCCESS;
+}
+
+} // namespace
+
 template <typename T>
 int contract_generic(T c_prefactor, ein_tensor_desc const &C, T *c, T ab_prefactor, ein_tensor_desc const &A, T const *a,
                      ein_tensor_desc const &B, T const *b, hipStream_t stream) {
@@ -815,6 +881,28 @@ int contract_generic(T c_prefactor, ein_tensor_desc const &C, T *c, T ab_prefact
         bool taken = false;
         EIN_TRY(contract_ttgt<T>(vb, vm, vn, vk, ab_prefactor, a, b, beta, c, stream, taken));
         if (taken) return EIN_SUCCESS;
+        // Small problems whose operands have a unit stride to read along: one wave per tile, in
+        // one launch also where C's unit stride is far from the tile's rows. To twice the
+        // tiles that a dense product would go to LDS with, for the gather's offsets cost the LDS kernel more:
+        // "pqrs <- pmrs, mq" FP64 with extents 24 11.0 -> 6.4 us, 32 (512 tiles) 13.6 -> 10.7,
+        // 36 (729) 21 -> 22; "mbej <- jnfb, mnef" with 12 and 40 88 -> 32, 16 and 48 (144, but
+        // 0.9 GFLOP) 56 -> 79. Without the unit stride the LDS kernel's reuse wins (200
+        // products of 20 x 20 x 500, one operand strided by the batch, 39 us, here 43).
+        if (t_route == EIN_ROUTE_AUTO && wave_small(M, N, K, NB, 2 * int64_t(num_cus()))) {
+            BuiltItem<T> it{};
+            EIN_TRY(build_wave<T>(vb, vm, vn, vk, a, b, c, ab_prefactor, beta, it));
+            auto unit = [](int64_t s) { return s == 1 || s == -1; };
+            if ((unit(it.w.sA) || unit(it.w.kA_in)) && (unit(it.w.tB) || unit(it.w.kB_in))) {
+                WaveLaunch<T> W{};
+                W.it    = it.w;
+                W.gm    = it.gm;
+                W.gn    = it.gn;
+                W.gk    = it.gk;
+                W.gb    = it.gb;
+                W.batch = it.batch;
+                return launch_wave<T, false>(W, stream);
+            }
+        }
         auto gm = order_and_fold(vm, 2, 0, 1);
         auto gn = order_and_fold(vn, 2, 0, 1);
         bool const a_i_fast = !gm.empty() && std::llabs(gm.back().s[0]) == 1;
@@ -1082,172 +1170,6 @@ int ein_contract_f32(float c_prefactor, const ein_tensor_desc *C, float *c, floa
 
 namespace ein {
 
-// One contraction as the wave kernel sees it: C[i,j] = alpha sum_p A[i,p] B[p,j] + beta C[i,j]
-// with element offsets from tables. C's unit stride, if it has one, is along i.
-template <typename T>
-struct WaveItem {
-    T const *A;
-    T const *B;
-    T *C;
-    T alpha, beta;
-    int64_t const *rowA, *rowC, *colB, *colC, *kA, *kB;
-    int64_t kA_in, kB_in; // stride per contraction step where k_mode says so
-    int64_t sA, sC, tB, tC; // strides of a single row digit (i) and column digit (j)
-    int32_t m, n, k;
-    int32_t k_mode; // 2: p * kA_in; 1: kA[p0] + (p - p0) * kA_in within 16 steps from p0; 0: kA[p]
-    int32_t m_lin, n_lin; // offsets of i (j) are i * sA, i * sC (j * tB, j * tC): no table
-};
-
-struct WaveTile {
-    int32_t item, tm, tn, pad; // tile (tm, tn) of the item, in units of its wave tile
-    int64_t oa, ob, oc;        // batch offsets
-};
-
-// Blocks of 16 rows (columns) in a wave tile: as many as the extent fills, up to most.
-__host__ __device__ __forceinline__ int wave_blocks(int64_t extent, int most) {
-    return extent <= 16 ? 1 : extent <= 32 || most < 4 ? 2 : 4;
-}
-
-// One wave's tile of 16*FM x 16*FN of C. The operands go from global memory straight to the
-// registers that feed the MFMA, 16 contraction steps at a time, the next 16 in flight during
-// the MFMAs: tiles of the small blocks that a grouped plan is made of share little that LDS
-// could hold for them, and without it there is no barrier, no padding to a slab layout, and
-// any alignment takes whole elements. Rows and columns outside the problem read its last one
-// and are not stored; steps beyond k are zeros in both operands. What bounds a plan of many
-// small items is the latency of a tile's first loads, so several waves share a SIMD and only
-// multi-digit indices go through tables. 1024 FP64 GEMMs with extents 4..512 took 1022 us with
-// 64/128 x 64 LDS tiles in a persistent walk, and take 133; 4096 of them 3.24 -> 0.51 ms
-// (FP32 1.20 -> 0.32); 2048 of 32 x 32 x 256 619 -> 53 us; 64 of 384^3 823 -> 198 (36 TFLOP/s).
-template <typename T, int FM, int FN>
-__device__ __forceinline__ void wave_tile(WaveItem<T> const &it, WaveTile const &e, int lane) {
-    int const r  = lane & 15;
-    int const q  = lane >> 4;
-    int const i0 = e.tm * 16 * FM, j0 = e.tn * 16 * FN;
-    int const k  = it.k;
-    T const *pa[FM];
-    T const *pb[FN];
-#pragma unroll
-    for (int a = 0; a < FM; ++a) {
-        int const i = i0 + a * 16 + r;
-        int const ic = i < it.m ? i : it.m - 1;
-        pa[a]        = it.A + e.oa + (it.m_lin ? ic * it.sA : it.rowA[ic]);
-    }
-#pragma unroll
-    for (int b = 0; b < FN; ++b) {
-        int const j = j0 + b * 16 + r;
-        int const jc = j < it.n ? j : it.n - 1;
-        pb[b]        = it.B + e.ob + (it.n_lin ? jc * it.tB : it.colB[jc]);
-    }
-    typename Mfma<T>::acc_t acc[FM][FN];
-#pragma unroll
-    for (int a = 0; a < FM; ++a)
-#pragma unroll
-        for (int b = 0; b < FN; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[a][b][v] = T(0);
-
-    struct Chunk {
-        T a[FM][4], b[FN][4];
-    };
-    // Which of a chunk's 16 steps lane group q feeds to the s-th MFMA does not matter as long as
-    // both operands agree. In a whole chunk it is V consecutive ones, so that an operand
-    // contiguous along k is read 16 bytes at a time (from any element: the hardware takes
-    // 16-byte loads at 4-byte alignment).
-    constexpr int V = 16 / int(sizeof(T));
-    typedef T vec_t __attribute__((ext_vector_type(V), aligned(sizeof(T))));
-    auto load = [&](int k0, Chunk &x) {
-        if (k0 + 16 <= k && it.k_mode != 0) {
-            int64_t const ba = it.k_mode == 2 ? k0 * it.kA_in : it.kA[k0];
-            int64_t const bb = it.k_mode == 2 ? k0 * it.kB_in : it.kB[k0];
-            auto operand = [&](auto const &ptr, int64_t base, int64_t step, auto &out, auto blocks) {
-                constexpr int NBK = decltype(blocks)::value;
-                if (step == 1) {
-#pragma unroll
-                    for (int h = 0; h < 4 / V; ++h)
-#pragma unroll
-                        for (int a = 0; a < NBK; ++a) {
-                            vec_t const t = *reinterpret_cast<vec_t const *>(ptr[a] + base + 4 * V * h + V * q);
-#pragma unroll
-                            for (int v = 0; v < V; ++v) out[a][V * h + v] = t[v];
-                        }
-                } else {
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        int64_t const o = base + (4 * V * (s / V) + V * q + s % V) * step;
-#pragma unroll
-                        for (int a = 0; a < NBK; ++a) out[a][s] = ptr[a][o];
-                    }
-                }
-            };
-            operand(pa, ba, it.kA_in, x.a, std::integral_constant<int, FM>{});
-            operand(pb, bb, it.kB_in, x.b, std::integral_constant<int, FN>{});
-        } else {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                if (k0 + 4 * s >= k) break;
-                int const p0     = k0 + 4 * s + q;
-                bool const in    = p0 < k;
-                int const p      = in ? p0 : k - 1;
-                int64_t const oa = it.k_mode == 2 ? p * it.kA_in : it.kA[p];
-                int64_t const ob = it.k_mode == 2 ? p * it.kB_in : it.kB[p];
-#pragma unroll
-                for (int a = 0; a < FM; ++a) {
-                    T const t  = pa[a][oa];
-                    x.a[a][s] = in ? t : T(0);
-                }
-#pragma unroll
-                for (int b = 0; b < FN; ++b) {
-                    T const t  = pb[b][ob];
-                    x.b[b][s] = in ? t : T(0);
-                }
-            }
-        }
-    };
-    auto multiply = [&](int k0, Chunk const &x) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (k0 + 4 * s >= k) break;
-#pragma unroll
-            for (int a = 0; a < FM; ++a)
-#pragma unroll
-                for (int b = 0; b < FN; ++b) acc[a][b] = Mfma<T>::mma(x.b[b][s], x.a[a][s], acc[a][b]);
-        }
-    };
-    Chunk x, y;
-    load(0, x);
-    for (int k0 = 0; k0 < k; k0 += 32) {
-        if (k0 + 16 < k) load(k0 + 16, y);
-        multiply(k0, x);
-        if (k0 + 16 >= k) break;
-        if (k0 + 32 < k) load(k0 + 32, x);
-        multiply(k0 + 16, y);
-    }
-
-    T *__restrict__ C = it.C + e.oc;
-#pragma unroll
-    for (int a = 0; a < FM; ++a) {
-        int const i = i0 + a * 16 + r;
-        if (i >= it.m) continue;
-        T *ci = C + (it.m_lin ? i * it.sC : it.rowC[i]);
-#pragma unroll
-        for (int b = 0; b < FN; ++b) {
-            int64_t oc[4];
-            T old[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                int const j = j0 + b * 16 + Mfma<T>::row(q, v);
-                int const jc = j < it.n ? j : it.n - 1;
-                oc[v]        = it.n_lin ? jc * it.tC : it.colC[jc];
-                old[v]      = it.beta != T(0) && j < it.n ? ci[oc[v]] : T(0);
-            }
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                if (j0 + b * 16 + Mfma<T>::row(q, v) < it.n)
-                    ci[oc[v]] = it.beta != T(0) ? it.alpha * acc[a][b][v] + it.beta * old[v] : it.alpha * acc[a][b][v];
-        }
-    }
-}
-
 // Grouped launch: one tile per wave, in list order (the hardware hands the next workgroup to
 // the next free slot, so the long tiles go first). MOST = 2 or 4 blocks of 16 rows per tile.
 template <typename T, int MOST>
@@ -1259,26 +1181,27 @@ __global__ __launch_bounds__(GEMM_THREADS, MOST == 2 ? 3 : 2) void grouped_wave_
     int const lane        = threadIdx.x & 63;
     WaveTile const e      = tiles[t];
     WaveItem<T> const &it = items[e.item];
+    TableOffsets<T> const off{it};
     int const fm = wave_blocks(it.m, MOST), fn = wave_blocks(it.n, 2);
     if constexpr (MOST == 4) {
         if (fm == 4) {
             if (fn == 2)
-                wave_tile<T, 4, 2>(it, e, lane);
+                wave_tile<4, 2>(it, e, off, lane);
             else
-                wave_tile<T, 4, 1>(it, e, lane);
+                wave_tile<4, 1>(it, e, off, lane);
             return;
         }
     }
     if (fm == 2) {
         if (fn == 2)
-            wave_tile<T, 2, 2>(it, e, lane);
+            wave_tile<2, 2>(it, e, off, lane);
         else
-            wave_tile<T, 2, 1>(it, e, lane);
+            wave_tile<2, 1>(it, e, off, lane);
     } else {
         if (fn == 2)
-            wave_tile<T, 1, 2>(it, e, lane);
+            wave_tile<1, 2>(it, e, off, lane);
         else
-            wave_tile<T, 1, 1>(it, e, lane);
+            wave_tile<1, 1>(it, e, off, lane);
     }
 }
 
@@ -1358,14 +1281,6 @@ ByteRange range_of(ein_tensor_desc const &d, void const *p, size_t elem) {
     return {base + uintptr_t(lo * int64_t(elem)), base + uintptr_t((hi + 1) * int64_t(elem))};
 }
 
-// One item: its problem with the index groups that its tables are built from.
-template <typename T>
-struct BuiltItem {
-    WaveItem<T> w;
-    IndexGroup gm, gn, gk, gb; // (A, C), (B, C), (A, B) and (A, B, C) strides
-    int64_t batch;
-};
-
 // Analyse one item (MFMA path for every size). kind: 0 = tiles to run, 1 = only a scale of C,
 // 2 = nothing to do.
 template <typename T>
@@ -1400,58 +1315,11 @@ int build_item(ein_contraction_item const &in, BuiltItem<T> &out, int &kind, boo
         kind = 1;
         return EIN_SUCCESS;
     }
-    int64_t M = total_of(vm), N = total_of(vn);
-    int64_t const K = total_of(vk), NB = total_of(vb);
+    int64_t const M = total_of(vm), N = total_of(vn), K = total_of(vk), NB = total_of(vb);
     if (M >= (int64_t{1} << 31) || N >= (int64_t{1} << 31) || K >= (int64_t{1} << 31) || NB >= (int64_t{1} << 31))
         return fail(EIN_ERROR_UNSUPPORTED, "grouped contraction: index range above 2^31");
-    // the lanes of a wave run along i when C is read and written: the side that holds C's
-    // unit stride becomes A
-    auto unit_in_c = [](std::vector<Digit> const &v) {
-        for (auto const &d : v)
-            if (std::llabs(d.s[1]) == 1) return true;
-        return false;
-    };
-    bool const swap = unit_in_c(vn) && !unit_in_c(vm);
-    T const *pa = static_cast<T const *>(in.a), *pb = static_cast<T const *>(in.b);
-    if (swap) {
-        std::swap(vm, vn);
-        std::swap(M, N);
-        std::swap(pa, pb);
-        for (auto &d : vk) std::swap(d.s[0], d.s[1]);
-        for (auto &d : vb) std::swap(d.s[0], d.s[1]);
-    }
-    auto gm = order_and_fold(vm, 2, 0, 1);
-    auto gn = order_and_fold(vn, 2, 0, 1);
-    bool const a_i_fast = !gm.empty() && std::llabs(gm.back().s[0]) == 1;
-    auto gk = a_i_fast ? order_and_fold(vk, 2, 1, 0) : order_and_fold(vk, 2, 0, 1);
-    auto gbv = order_and_fold(vb, 3, 2, 0);
-    EIN_TRY(fill_group(out.gm, gm, 2));
-    EIN_TRY(fill_group(out.gn, gn, 2));
-    EIN_TRY(fill_group(out.gk, gk, 2));
-    EIN_TRY(fill_group(out.gb, gbv, 3));
-    out.batch       = NB;
-    WaveItem<T> &w  = out.w;
-    w        = WaveItem<T>{};
-    w.A      = pa;
-    w.B      = pb;
-    w.C      = static_cast<T *>(in.c);
-    w.alpha  = T(in.ab_prefactor);
-    w.beta   = c_repeats ? T(1) : T(in.c_prefactor);
-    w.m      = int32_t(M);
-    w.n      = int32_t(N);
-    w.k      = int32_t(K);
-    // one digit: affine over all of k. Otherwise affine within 16 steps where the innermost
-    // digit's extent is a multiple of 16 (chunks start at multiples of 16)
-    w.k_mode = gk.size() <= 1 ? 2 : gk.back().e % 16 == 0 ? 1 : 0;
-    w.kA_in  = gk.empty() ? 0 : gk.back().s[0];
-    w.kB_in  = gk.empty() ? 0 : gk.back().s[1];
-    w.m_lin  = gm.size() <= 1;
-    w.n_lin  = gn.size() <= 1;
-    w.sA     = gm.empty() ? 0 : gm.back().s[0];
-    w.sC     = gm.empty() ? 0 : gm.back().s[1];
-    w.tB     = gn.empty() ? 0 : gn.back().s[0];
-    w.tC     = gn.empty() ? 0 : gn.back().s[1];
-    return EIN_SUCCESS;
+    return build_wave<T>(vb, vm, vn, vk, static_cast<T const *>(in.a), static_cast<T const *>(in.b), static_cast<T *>(in.c),
+                         T(in.ab_prefactor), c_repeats ? T(1) : T(in.c_prefactor), out);
 }
 
 // The result equals running the items one after another in list order. Item j depends on

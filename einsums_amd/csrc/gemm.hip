@@ -17,6 +17,7 @@
 
 #include "gemm.hpp"
 #include "tile_engine.hpp"
+#include "wave_tile.hpp"
 
 namespace ein {
 
@@ -347,13 +348,31 @@ TuneKey tune_key(GemmProblem<T> const &P) {
     return TuneKey{int(sizeof(T)), P.m, P.n, P.k, P.batch, P.a_sk == 1 ? 1 : 0, P.b_sk == 1 ? 1 : 0};
 }
 
+// Products for one wave per tile (wave_tile.hpp), without LDS: small ones, and those with a
+// side of at most 32 and at most 1024 steps, where an LDS tile is at least half padding and the
+// time is the reading of the long side. Measured FP64 (FP32): 1000000 x 16 x 16 78 -> 44 us (52 ->
+// 24), 100000 x 32 x 32 20.3 -> 18.8 (18 -> 9.7), 300000 x 32 x 128 123 -> 103 (70 -> 50), 30000 x
+// 32 x 1000 91 -> 62 (54 -> 46), 4096 products of 32^3 32 -> 23 (26 -> 12.6), 10000 of 16^3 48 ->
+// 13 (31 -> 7); but 10000 x 32 x 4000 115 and here 213, 1000 products of 48^3 14.0 and here 17.9.
+bool prefer_wave(int64_t m, int64_t n, int64_t k, int64_t batch) {
+    if (!wave_fits(m, n, k, batch)) return false;
+    return wave_small(m, n, k, batch, num_cus()) || ((m <= 32 || n <= 32) && k <= 1024);
+}
+
 // Candidate configurations: tile shape x schedule (hybrid stream-K or data-parallel) x
 // workgroups per CU the schedule plans for (all that fit, or one).
 // krow_both: both operands contiguous along k (row-major LDS staging), the case the 96 x 96
 // tile is built for (576 = 6 x 96: the Wmnij GEMM at o=24 has no ragged tiles).
 // fp32: adds the 256 x 128 tile, which only FP32's accumulators leave registers for.
-std::vector<GemmConfig> tune_candidates(bool krow_both, bool fp32) {
+// wave: adds one wave per tile, written as 16 x 16.
+std::vector<GemmConfig> tune_candidates(bool krow_both, bool fp32, bool wave) {
     std::vector<GemmConfig> c;
+    if (wave) {
+        GemmConfig g;
+        g.bm = 16;
+        g.bn = 16;
+        c.push_back(g);
+    }
     if (fp32)
         for (int dp : {0, 1}) {
             GemmConfig g;
@@ -427,7 +446,7 @@ int tune_gemm(GemmProblem<T> const &P, hipStream_t stream, GemmConfig *best) {
     Q.c_sn           = P.m;
     Q.c_sb           = P.m * P.n;
     Q.beta           = P.beta;
-    std::vector<GemmConfig> const cands = tune_candidates(krow_both(P), sizeof(T) == 4);
+    std::vector<GemmConfig> const cands = tune_candidates(krow_both(P), sizeof(T) == 4, prefer_wave(P.m, P.n, P.k, P.batch));
     std::vector<float> best_of(cands.size(), 0.f);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int st = EIN_SUCCESS;
@@ -506,7 +525,7 @@ int gemm_strided_impl(GemmProblem<T> P, GemmConfig const *force, hipStream_t str
             if (ws_bytes != nullptr) {
                 // an untuned key in tuning mode may run any candidate: report the largest need
                 size_t most = 0;
-                for (GemmConfig const &c : tune_candidates(krow_both(P), sizeof(T) == 4)) {
+                for (GemmConfig const &c : tune_candidates(krow_both(P), sizeof(T) == 4, prefer_wave(P.m, P.n, P.k, P.batch))) {
                     size_t b = 0;
                     EIN_TRY(gemm_strided_impl<T>(P, &c, stream, &b));
                     most = std::max(most, b);
@@ -523,6 +542,33 @@ int gemm_strided_impl(GemmProblem<T> P, GemmConfig const *force, hipStream_t str
         }
     }
     if (have_tuned) force = &tuned;
+    bool const wave = force ? force->bm == 16 : prefer_wave(P.m, P.n, P.k, P.batch);
+    if (wave) {
+        if (!wave_fits(P.m, P.n, P.k, P.batch))
+            return fail(EIN_ERROR_UNSUPPORTED, "gemm: problem too large for one wave per tile");
+        if (ws_bytes != nullptr) return EIN_SUCCESS;
+        WaveLaunch<T> W{};
+        W.it.A      = P.A;
+        W.it.B      = P.B;
+        W.it.C      = P.C;
+        W.it.alpha  = P.alpha;
+        W.it.beta   = P.beta;
+        W.it.kA_in  = P.a_sk;
+        W.it.kB_in  = P.b_sk;
+        W.it.sA     = P.a_sm;
+        W.it.sC     = P.c_sm;
+        W.it.tB     = P.b_sn;
+        W.it.tC     = P.c_sn;
+        W.it.m      = int32_t(P.m);
+        W.it.n      = int32_t(P.n);
+        W.it.k      = int32_t(P.k);
+        W.it.k_mode = 2;
+        W.a_sb      = P.a_sb;
+        W.b_sb      = P.b_sb;
+        W.c_sb      = P.c_sb;
+        W.batch     = P.batch;
+        return launch_wave<T, true>(W, stream);
+    }
     GemmConfig cfg = force ? *force : choose_gemm_config(P.m, P.n, P.k, P.batch, int(sizeof(T)));
     if (!force && cfg.bm == 128 && cfg.bn == 64) {
         // few tiles with both operands staged row-major (contiguous along k): 64 x 64
@@ -823,8 +869,9 @@ int ein_gemm_tuning_load(const char *path) {
         long long m, n, k, b;
         if (std::sscanf(line, "%d %lld %lld %lld %lld %d %d : %d %d %d %d", &eb, &m, &n, &k, &b, &ak, &bk, &bm, &bn, &dp,
                         &bpc) != 11 ||
-            (eb != 4 && eb != 8) || (bm != 64 && bm != 96 && bm != 128 && (bm != 256 || eb != 4 || bn != 128)) ||
-            (bn != 64 && bn != 96 && bn != 128) || (bm == 96) != (bn == 96) ||
+            (eb != 4 && eb != 8) || (bm != 16 && bm != 64 && bm != 96 && bm != 128 && (bm != 256 || eb != 4 || bn != 128)) ||
+            (bn != 16 && bn != 64 && bn != 96 && bn != 128) || (bm == 16) != (bn == 16) || (bm == 96) != (bn == 96) ||
+            (bm == 16 && !ein::wave_fits(m, n, k, b)) ||
             dp < 0 || dp > 2 || bpc < 0 ||
             m <= 0 || n <= 0 || k <= 0 || b <= 0) {
             std::fclose(f);
