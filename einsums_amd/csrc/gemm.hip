@@ -22,12 +22,20 @@
 namespace ein {
 
 // Operand slabs go global -> LDS by DMA (tile_engine.hpp); AKG / BKG select the
-// row-major (KROW) LDS layout for an operand contiguous along k, AW / BW the 16-byte DMA.
+// row-major (KROW) LDS layout for an operand contiguous along k, AW / BW the 16-byte DMA. An
+// operand without it goes through registers, 16 bytes at a time all the same: what a dword DMA
+// costs is four times the instructions. 1531 x 1013 x 2047 FP64 NT 165 -> 142 us, 4095^3 2852 ->
+// 2353 (58 TFLOP/s), 625 x 625 x 8649 218 -> 166; FP32 841 x 841 x 7921 TN 175 -> 140.
 template <typename T, int BM, int BN, int BK, bool AKG, bool AW, bool BKG, bool BW>
 __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_dense_kernel(GemmProblem<T> P) {
     using Cfg = TileCfg<T, BM, BN, BK>;
-    using LA  = SlabLayout<T, BM, BK, AKG, AW>;
-    using LB  = SlabLayout<T, BN, BK, BKG, BW>;
+    // through registers where the DMA would be dword wide and the chunks' layout is realisable
+    // (the 256-row tile has no registers left: FP32 4095^3 NT 1286 us, with it 2122)
+    constexpr bool AR = !AW && BM <= 128 && SlabLayout<T, BM, BK, AKG, true>::VALID;
+    constexpr bool BR = !BW && BM <= 128 && SlabLayout<T, BN, BK, BKG, true>::VALID;
+    constexpr bool AL = AW || AR, BL = BW || BR;
+    using LA  = SlabLayout<T, BM, BK, AKG, AL>;
+    using LB  = SlabLayout<T, BN, BK, BKG, BL>;
     __shared__ __attribute__((aligned(16))) T As[2 * LA::SIZE];
     __shared__ __attribute__((aligned(16))) T Bs[2 * LB::SIZE];
 
@@ -35,7 +43,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_dense_kernel(GemmProblem
     int const lane = tid & 63;
     // wave-uniform, so per-instruction contraction offsets of the DMA stay scalar (not for
     // the dword row-major staging, where it makes the compiler keep more lane offsets live)
-    constexpr bool dword_krow = (AKG && !AW) || (BKG && !BW);
+    constexpr bool dword_krow = (AKG && !AL) || (BKG && !BL);
     int const wave = dword_krow ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
     int const wm   = wave & 1;
     int const wn   = wave >> 1;
@@ -74,14 +82,28 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_dense_kernel(GemmProblem
         // both operands' slabs at k0; without bounds checks when tile and slab are inside
         // (not for the dword row-major staging, whose registers a second copy would spill)
         bool const full_mn = !dword_krow && mrem >= BM && nrem >= BN;
-        auto dma_both      = [&](T *Ad, T *Bd, int64_t k0) {
-            if (full_mn && k0 + BK <= kend) {
-                dma_slab<T, BM, BK, AKG, AW, false>(Ab, Ad, wave, lane, k0, offA);
-                dma_slab<T, BN, BK, BKG, BW, false>(Bb, Bd, wave, lane, k0, offB);
-            } else {
-                dma_slab<T, BM, BK, AKG, AW>(Ab, Ad, wave, lane, k0, offA);
-                dma_slab<T, BN, BK, BKG, BW>(Bb, Bd, wave, lane, k0, offB);
-            }
+        RegSlab<T, BM, BK, AKG> ra;
+        RegSlab<T, BN, BK, BKG> rb;
+        auto stage_in = [&](T *Ad, T *Bd, int64_t k0, auto check) {
+            constexpr bool CHECK = decltype(check)::value;
+            if constexpr (AR)
+                ra.template load<CHECK>(Ab + k0 * P.a_sk, wave, lane, P.a_sm, P.a_sk, mrem, kend - k0);
+            else
+                dma_slab<T, BM, BK, AKG, AL, CHECK>(Ab, Ad, wave, lane, k0, offA);
+            if constexpr (BR)
+                rb.template load<CHECK>(Bb + k0 * P.b_sk, wave, lane, P.b_sn, P.b_sk, nrem, kend - k0);
+            else
+                dma_slab<T, BN, BK, BKG, BL, CHECK>(Bb, Bd, wave, lane, k0, offB);
+        };
+        auto dma_both = [&](T *Ad, T *Bd, int64_t k0) {
+            if (full_mn && k0 + BK <= kend)
+                stage_in(Ad, Bd, k0, std::false_type{});
+            else
+                stage_in(Ad, Bd, k0, std::true_type{});
+        };
+        auto commit = [&](T *Ad, T *Bd) {
+            if constexpr (AR) ra.store(Ad, wave, lane);
+            if constexpr (BR) rb.store(Bd, wave, lane);
         };
 
         WaveAcc<T, Cfg::FM, Cfg::FN> acc;
@@ -90,15 +112,19 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void gemm_dense_kernel(GemmProblem
         int64_t const kbeg   = int64_t(s0) * BK;
         __syncthreads(); // LDS of the previous segment no longer read
         dma_both(As, Bs, kbeg);
+        commit(As, Bs);
         for (int64_t sl = 0; sl < nslabs; ++sl) {
             int const buf = int(sl & 1);
             dma_wait_all();
             auto next_dma = [&](T *An, T *Bn) {
                 if (sl + 1 < nslabs) dma_both(An, Bn, kbeg + (sl + 1) * BK);
             };
-            mfma_slab_lds<T, BM, BN, BK, AKG, AW, BKG, BW>(As + buf * LA::SIZE, Bs + buf * LB::SIZE,
+            auto next_commit = [&](T *An, T *Bn) {
+                if (sl + 1 < nslabs) commit(An, Bn);
+            };
+            mfma_slab_lds<T, BM, BN, BK, AKG, AL, BKG, BL>(As + buf * LA::SIZE, Bs + buf * LB::SIZE,
                                                            As + (buf ^ 1) * LA::SIZE, Bs + (buf ^ 1) * LB::SIZE, acc, wm,
-                                                           wn, lane, next_dma);
+                                                           wn, lane, next_dma, next_commit);
         }
 
         // Lane coordinates made opaque per segment so the compiler does not hoist the
@@ -229,7 +255,11 @@ namespace {
 
 template <typename T, int BM, int BN, int BK, bool AKG, bool AW, bool BKG, bool BW>
 void const *dense_kernel_ptr() {
-    if constexpr (SlabLayout<T, BM, BK, AKG, AW>::VALID && SlabLayout<T, BN, BK, BKG, BW>::VALID)
+    constexpr bool regs = BM <= 128;
+    constexpr bool a_ok = SlabLayout<T, BM, BK, AKG, AW>::VALID || (!AW && regs && SlabLayout<T, BM, BK, AKG, true>::VALID);
+    constexpr bool b_ok = SlabLayout<T, BN, BK, BKG, BW>::VALID || (!BW && regs && SlabLayout<T, BN, BK, BKG, true>::VALID);
+    // 256 rows a dword at a time along k: never launched (rows_256)
+    if constexpr (a_ok && b_ok && (regs || !AKG || AW))
         return reinterpret_cast<void const *>(&gemm_dense_kernel<T, BM, BN, BK, AKG, AW, BKG, BW>);
     else
         return nullptr;
@@ -577,7 +607,15 @@ int gemm_strided_impl(GemmProblem<T> P, GemmConfig const *force, hipStream_t str
         bool const b_krow = choose_staging<T>(64, P.b_sn, P.b_sk, P.b_sb, P.batch, P.n, P.k, P.B).krow;
         if (a_krow && b_krow) cfg.bm = 64;
     }
-    if (sizeof(T) == 4 && !force && cfg.bm == 128 && cfg.bn == 128 &&
+    // The 256-row tile stages an A that is contiguous along k by 16-byte DMA or not at all: its
+    // registers are all taken, and a dword at a time costs more than 128 rows through registers
+    // (FP32 4096 x 4096 x 4095 NT 1284 us, so 1198; 4095^3 TT 1629, so 1269).
+    auto rows_256 = [&] {
+        OperandStaging const sa = choose_staging<T>(256, P.a_sm, P.a_sk, P.a_sb, P.batch, P.m, P.k, P.A);
+        return !sa.krow || sa.wide;
+    };
+    if (force && cfg.bm == 256 && !rows_256()) cfg.bm = 128;
+    if (sizeof(T) == 4 && !force && cfg.bm == 128 && cfg.bn == 128 && rows_256() &&
         ceil_div(P.m, 256) * ceil_div(P.n, 128) * P.batch >= 2 * int64_t(num_cus())) {
         // FP32 slabs of 128 x 128 are half as long in time as FP64's, and what they stage per
         // MFMA is what holds them back (without the staging 140 TFLOP/s, with it 119): from two

@@ -132,6 +132,51 @@ __device__ __forceinline__ void dma_slab(T const *__restrict__ base, T *lds, int
     }
 }
 
+// Staging through registers, for an operand that the 16-byte DMA cannot take (its chunks are
+// not 16-byte aligned, or an edge of the problem cuts one): the same chunks in the same layout,
+// read by ordinary loads, which take 16 bytes from any element, and written to LDS once the
+// slab before is multiplied. A dword DMA moves a quarter per instruction.
+template <typename T, int ROWS, int BK, bool KROW>
+struct RegSlab {
+    using L                 = SlabLayout<T, ROWS, BK, KROW, true>;
+    static constexpr int CE = L::CE;
+    typedef T vec_t __attribute__((ext_vector_type(CE)));
+    typedef vec_t any_vec_t __attribute__((aligned(sizeof(T))));
+    vec_t v[L::INS_PER_WAVE];
+
+    // base: element (0, 0) of the slab; rows and ks: what is left of the problem from there.
+    // With CHECK false the slab is inside.
+    template <bool CHECK>
+    __device__ __forceinline__ void load(T const *__restrict__ base, int wave, int lane, int64_t s_row, int64_t s_k,
+                                         int64_t rows, int64_t ks) {
+        int64_t const step = KROW ? s_k : s_row;
+#pragma unroll
+        for (int x = 0; x < L::INS_PER_WAVE; ++x) {
+            int row, k, h;
+            L::lane_elem(wave, x, lane, row, k, h);
+            if constexpr (KROW) asm volatile("" : "+v"(row)); // as in dma_slab
+            T const *src       = base + (row * s_row + k * s_k);
+            int64_t const left = KROW ? ks - k : rows - row;
+            bool const in      = !CHECK || (KROW ? row < rows : k < ks);
+            if (step == 1 && (!CHECK || (in && left >= CE))) {
+                v[x] = *reinterpret_cast<any_vec_t const *>(src);
+            } else {
+#pragma unroll
+                for (int e = 0; e < CE; ++e) {
+                    T t = T(0);
+                    if (in && (!CHECK || e < left)) t = src[e * step];
+                    v[x][e] = t;
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ void store(T *lds, int wave, int lane) const {
+#pragma unroll
+        for (int x = 0; x < L::INS_PER_WAVE; ++x)
+            *reinterpret_cast<vec_t *>(reinterpret_cast<uint32_t *>(lds) + L::ins_base_dw(wave, x) + lane * L::VW) = v[x];
+    }
+};
+
 // MFMA work of one slab from LDS, with the fragments of step kk+4 read while the MFMAs of
 // step kk run. As/Bs are the slab buffers of A (rows along i) and B (rows along j), An/Bn
 // the buffers the next slab's DMA fills: `dma(An, Bn)` runs after the first fragments are
@@ -139,11 +184,17 @@ __device__ __forceinline__ void dma_slab(T const *__restrict__ base, T *lds, int
 // All four are restrict parameters of this (inlined) function: the compiler then knows
 // that the fragment reads cannot alias the in-flight DMA and does not wait for it before
 // every LDS read of the slab.
-template <typename T, int BM, int BN, int BK, bool AKG, bool AW, bool BKG, bool BW, typename Dma>
+// `commit(An, Bn)` runs after the last MFMA: it stores what `dma` left in registers.
+struct NoCommit {
+    template <typename T>
+    __device__ __forceinline__ void operator()(T *, T *) const {}
+};
+
+template <typename T, int BM, int BN, int BK, bool AKG, bool AW, bool BKG, bool BW, typename Dma, typename Commit = NoCommit>
 __device__ __forceinline__ void mfma_slab_lds(T const *__restrict__ As, T const *__restrict__ Bs, T *__restrict__ An,
                                               T *__restrict__ Bn,
                                               WaveAcc<T, TileCfg<T, BM, BN, BK>::FM, TileCfg<T, BM, BN, BK>::FN> &acc,
-                                              int wm, int wn, int lane, Dma const &dma) {
+                                              int wm, int wn, int lane, Dma const &dma, Commit const &commit = Commit{}) {
     using Cfg = TileCfg<T, BM, BN, BK>;
     using LA  = SlabLayout<T, BM, BK, AKG, AW>;
     using LB  = SlabLayout<T, BN, BK, BKG, BW>;
@@ -170,6 +221,7 @@ __device__ __forceinline__ void mfma_slab_lds(T const *__restrict__ As, T const 
         // 4096^3..16384^2; the wave-priority alternative measured -2%)
         __builtin_amdgcn_iglp_opt(0);
     }
+    commit(An, Bn);
 }
 
 // Whether a tile of `rows` rows has a k-major layout for 16-byte DMA: an instruction covers part
