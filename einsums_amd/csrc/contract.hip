@@ -299,19 +299,10 @@ template <typename T, int BM, int BN>
 __global__ __launch_bounds__(256) void gather_streamk_fixup(GatherProblem<T> P) {
     StreamK const &sk = P.sk;
     uint64_t const t  = uint64_t(sk.dp_tiles) + blockIdx.y;
-    uint64_t g0, g1;
-    sk_owners(sk, t, g0, g1);
-    if (g0 == g1) return;
-    int const e0     = int(blockIdx.x) * 256 + int(threadIdx.x);
-    int const stride = int(gridDim.x) * 256;
+    int const e0      = int(blockIdx.x) * 256 + int(threadIdx.x);
+    int const stride  = int(gridDim.x) * 256;
     T sum[FIXUP_EPT];
-#pragma unroll
-    for (int x = 0; x < FIXUP_EPT; ++x) sum[x] = T(0);
-    for (uint64_t g = g0; g <= g1; ++g) {
-        T const *__restrict__ pc = P.partial + sk_slot(sk, g, t) * (BM * BN);
-#pragma unroll
-        for (int x = 0; x < FIXUP_EPT; ++x) sum[x] += pc[e0 + x * stride];
-    }
+    if (!sk_sum_pieces<T, BM * BN>(sk, P.partial, t, e0, stride, sum)) return;
     uint32_t const tiles_mn = P.tiles_m * P.tiles_n;
     uint32_t const bz       = uint32_t(t / tiles_mn);
     uint32_t tm, tn;
@@ -637,13 +628,18 @@ int pack_digits(T const *src, std::vector<std::pair<std::vector<Digit> const *, 
 // the dense MFMA GEMM (or the split-precision GEMM when that mode is on), and an output
 // that does not fold is formed in a dense buffer X ([batch][N][M], M fastest) and added
 // into C by the permute. Digit orders are chosen to fold as much as possible. The route
-// is taken (`taken` = true) when its extra traffic and launches cost less than the
-// measured gap between the gather GEMM and the dense GEMM (the gather kernel takes about
-// 1.45x the dense kernel's time at 2304^3 FP64 on MI355X).
+// is taken (`taken` = true) when nothing is packed, or when packing, dense product and staging
+// are put below gather_us, the estimate of the gather GEMM (0: only if nothing is packed).
+// Fitted to "mbej <- jnfb, mnef" (o 9..32, v 43..104) and "pqrs <- pmrs, mq" (36..100) in FP64 and
+// FP32: over 44 of them the choice loses at most 6% against the better route, where 0.45 of
+// the dense product's time as the line for the extra traffic took the gather for 17 x 51 (FP64 145 us,
+// packed 66), 13 x 77 (207, 92), 20 x 60 (133, 105), 16 x 64 (82, 71).
+constexpr double GATHER_SLOWER[] = {1.65, 1.1}, GATHER_UNALIGNED[] = {1.5, 1.0}; // FP64, FP32
+
 template <typename T>
 int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, std::vector<Digit> const &vn,
-                  std::vector<Digit> const &vk, T alpha, T const *a, T const *b, T beta, T *c, hipStream_t stream,
-                  bool &taken) {
+                  std::vector<Digit> const &vk, T alpha, T const *a, T const *b, T beta, T *c, double gather_us,
+                  hipStream_t stream, bool &taken) {
     taken = false;
     if (t_route == EIN_ROUTE_GATHER) return EIN_SUCCESS;
     bool const forced = t_route == EIN_ROUTE_TTGT;
@@ -679,9 +675,24 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
                 if (best.moved < 0.0 || ch.moved < best.moved) best = ch;
             }
     int const launches   = int(!best.a_ok) + int(!best.b_ok) + int(!best.c_ok);
-    double const t_gemm  = 2.0 * double(NB) * M * N * K / (sizeof(T) == 8 ? 55e12 : 100e12);
-    double const t_extra = 2.0 * sizeof(T) * best.moved / 4e12 + 5e-6 * launches;
-    if (!forced && t_extra >= 0.45 * t_gemm) return EIN_SUCCESS;
+    if (!forced && launches > 0) {
+        bool below;
+        if (sizeof(T) == 8 && gemm_split_on()) {
+            // the split product replaces the dense one: the choice that goes with it
+            double const t_gemm  = 2.0 * double(NB) * M * N * K / 55e12;
+            double const t_extra = 2.0 * sizeof(T) * best.moved / 4e12 + 5e-6 * launches;
+            below                = t_extra < 0.45 * t_gemm;
+        } else {
+            auto unaligned = [&](bool ok, int64_t const *s, int64_t rows, T const *ptr) {
+                return !(ok ? choose_staging<T>(128, s[1], s[2], s[0], NB, rows, K, ptr).wide : K * int64_t(sizeof(T)) % 16 == 0);
+            };
+            int const ua = unaligned(best.a_ok, best.as, M, a), ub = unaligned(best.b_ok, best.bs, N, b);
+            double const dense = gemm_time_us(M, N, K, NB, int(sizeof(T)), true, ua + ub);
+            double const extra = 2e6 * sizeof(T) * best.moved / 5e12 + (sizeof(T) == 8 ? 4.0 : 5.0) * launches;
+            below              = dense + extra < 0.95 * gather_us;
+        }
+        if (!below) return EIN_SUCCESS;
+    }
 
     auto align = [](size_t x) { return (x + 255) / 256 * 256; };
     size_t const a_bytes = best.a_ok ? 0 : align(size_t(NB * M * K) * sizeof(T));
@@ -692,8 +703,10 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
     if (total > 0) {
         // under stream capture the buffer must already exist; otherwise the gather runs
         if (!forced && stream_capturing(stream) && !workspace_fits(stream, 1, total)) return EIN_SUCCESS;
-        void *p = nullptr;
-        EIN_TRY(workspace_slot(stream, 1, total, &p));
+        void *p      = nullptr;
+        int const st = workspace_slot(stream, 1, total, &p);
+        if (st == EIN_ERROR_ALLOC && !forced) return EIN_SUCCESS; // the gather needs no packed copies
+        if (st != EIN_SUCCESS) return st;
         ws = static_cast<char *>(p);
     }
     taken = true;
@@ -879,20 +892,27 @@ int contract_generic(T c_prefactor, ein_tensor_desc const &C, T *c, T ab_prefact
 
     if (use_mfma) {
         bool taken = false;
-        EIN_TRY(contract_ttgt<T>(vb, vm, vn, vk, ab_prefactor, a, b, beta, c, stream, taken));
-        if (taken) return EIN_SUCCESS;
+        bool small = t_route == EIN_ROUTE_AUTO && wave_small(M, N, K, NB, 2 * int64_t(num_cus()), 3e8);
+        if (small) {
+            EIN_TRY(contract_ttgt<T>(vb, vm, vn, vk, ab_prefactor, a, b, beta, c, 0.0, stream, taken));
+            if (taken) return EIN_SUCCESS;
+        }
         // Small problems whose operands have a unit stride to read along: one wave per tile, in
         // one launch also where C's unit stride is far from the tile's rows. To twice the
         // tiles that a dense product would go to LDS with, for the gather's offsets cost the LDS kernel more:
         // "pqrs <- pmrs, mq" FP64 with extents 24 11.0 -> 6.4 us, 32 (512 tiles) 13.6 -> 10.7,
         // 36 (729) 21 -> 22; "mbej <- jnfb, mnef" with 12 and 40 88 -> 32, 16 and 48 (144, but
-        // 0.9 GFLOP) 56 -> 79. Without the unit stride the LDS kernel's reuse wins (200
+        // 0.9 GFLOP) 56 -> 79. Beyond 0.3 GFLOP packing and a dense product pass it (518 x 418 x 825
+        // FP64 39 us, here 46), in FP32 from 0.1 if every step's offset is decoded (264 x 261 x 962
+        // 23 us, here 39). Without the unit stride the LDS kernel's reuse wins (200
         // products of 20 x 20 x 500, one operand strided by the batch, 39 us, here 43).
-        if (t_route == EIN_ROUTE_AUTO && wave_small(M, N, K, NB, 2 * int64_t(num_cus()))) {
+        if (small) {
             BuiltItem<T> it{};
             EIN_TRY(build_wave<T>(vb, vm, vn, vk, a, b, c, ab_prefactor, beta, it));
             auto unit = [](int64_t s) { return s == 1 || s == -1; };
-            if ((unit(it.w.sA) || unit(it.w.kA_in)) && (unit(it.w.tB) || unit(it.w.kB_in))) {
+            small     = (unit(it.w.sA) || unit(it.w.kA_in)) && (unit(it.w.tB) || unit(it.w.kB_in)) &&
+                    (sizeof(T) == 8 || it.w.k_mode != 0 || wave_small(M, N, K, NB, 2 * int64_t(num_cus()), 1e8));
+            if (small) {
                 WaveLaunch<T> W{};
                 W.it    = it.w;
                 W.gm    = it.gm;
@@ -918,6 +938,23 @@ int contract_generic(T c_prefactor, ein_tensor_desc const &C, T *c, T ab_prefact
         // the batch) and added into C by the LDS-tiled permute, whose reads and writes are
         // both coalesced.
         bool const stage = std::llabs(gm.back().s[1]) >= 16 && int(gm.size() + gn.size() + gbv.size()) <= EIN_MAX_RANK;
+        GemmConfig cfg = choose_gemm_config(M, N, K, NB, int(sizeof(T)));
+        int const bm   = cfg.bm == 128 ? 128 : 64;
+        int const bn   = cfg.bn == 128 ? 128 : 64;
+        OperandStaging sa{!a_fast, false}, sb{!b_j_fast, false};
+        sa.wide = a_fast ? (kmajor_wide<T>(bm) && gather_wide_ok<T>(gm, 0, gk, 0, gbv, 0, a))
+                         : gather_wide_ok<T>(gk, 0, gm, 0, gbv, 0, a);
+        sb.wide = b_j_fast ? (kmajor_wide<T>(bn) && gather_wide_ok<T>(gn, 0, gk, 1, gbv, 1, b))
+                           : gather_wide_ok<T>(gk, 1, gn, 0, gbv, 1, b);
+        if (!small && t_route != EIN_ROUTE_GATHER) {
+            // slabs of the gather take GATHER_SLOWER times the dense kernel's and more for each
+            // operand copied a dword at a time; its tables and its staging are launches
+            double const slower = GATHER_SLOWER[sizeof(T) == 4] + GATHER_UNALIGNED[sizeof(T) == 4] * ((sa.wide ? 0 : 1) + (sb.wide ? 0 : 1));
+            double const us     = 4.0 + gemm_time_us(M, N, K, NB, int(sizeof(T)), cfg, slower) +
+                              (stage ? 4.0 + 2e6 * sizeof(T) * double(M) * double(N) * double(NB) / 5e12 : 0.0);
+            EIN_TRY(contract_ttgt<T>(vb, vm, vn, vk, ab_prefactor, a, b, beta, c, us, stream, taken));
+            if (taken) return EIN_SUCCESS;
+        }
         std::vector<Digit> const gm_c = gm, gn_c = gn, gb_c = gbv; // C strides
         if (stage) {
             int64_t pv = 1;
@@ -949,18 +986,10 @@ int contract_generic(T c_prefactor, ein_tensor_desc const &C, T *c, T ab_prefact
         P.C     = c;
         P.alpha = ab_prefactor;
         P.beta  = beta;
-        GemmConfig cfg = choose_gemm_config(M, N, K, NB, int(sizeof(T)));
-        int const bm   = cfg.bm == 128 ? 128 : 64;
-        int const bn   = cfg.bn == 128 ? 128 : 64;
         P.tiles_m      = uint32_t(ceil_div(M, bm));
         P.tiles_n      = uint32_t(ceil_div(N, bn));
         uint64_t tiles   = uint64_t(P.tiles_m) * P.tiles_n * uint64_t(NB);
         if (tiles > 0x7fffffffu) return fail(EIN_ERROR_UNSUPPORTED, "contraction tile grid too large");
-        OperandStaging sa{!a_fast, false}, sb{!b_j_fast, false};
-        sa.wide = a_fast ? (kmajor_wide<T>(bm) && gather_wide_ok<T>(gm, 0, gk, 0, gbv, 0, a))
-                         : gather_wide_ok<T>(gk, 0, gm, 0, gbv, 0, a);
-        sb.wide = b_j_fast ? (kmajor_wide<T>(bn) && gather_wide_ok<T>(gn, 0, gk, 1, gbv, 1, b))
-                           : gather_wide_ok<T>(gk, 1, gn, 0, gbv, 1, b);
         void const *kern = bm == 128 && bn == 128 ? gather_kernel_for<T, 128, 128>(sa, sb)
                            : bm == 128            ? gather_kernel_for<T, 128, 64>(sa, sb)
                                                   : gather_kernel_for<T, 64, 64>(sa, sb);
@@ -989,7 +1018,7 @@ int contract_generic(T c_prefactor, ein_tensor_desc const &C, T *c, T ab_prefact
         }
         void *args[] = {&P};
         EIN_HIP_CHECK(hipLaunchKernel(kern, dim3(P.sk.grid), dim3(GEMM_THREADS), args, 0, stream));
-        if (P.sk.units != 0) {
+        if (sk_cuts(P.sk)) {
             if (bm == 128 && bn == 128)
                 gather_streamk_fixup<T, 128, 128><<<sk_fixup_grid(P.sk, 128 * 128), 256, 0, stream>>>(P);
             else if (bm == 128)

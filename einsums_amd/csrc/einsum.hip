@@ -28,6 +28,8 @@ thread_local int t_split_type   = EIN_SLICE_BF16;
 
 } // namespace
 
+bool gemm_split_on() { return t_split_slices != 0; }
+
 template <typename T>
 int gemm_dispatch(GemmProblem<T> const &P, hipStream_t stream) {
     if constexpr (std::is_same_v<T, double>) {

@@ -13,6 +13,9 @@ template <typename T>
 int einsum_execute(int alg, T cp, ein_tensor_desc const &C, T *c, T abp, ein_tensor_desc const &A, T const *a,
                    ein_tensor_desc const &B, T const *b, int32_t *used, hipStream_t stream);
 
+// Whether FP64 products that map to a GEMM run as split ones on this thread.
+bool gemm_split_on();
+
 // GEMM of a GEMM-mapped einsum: the split-precision GEMM when this thread's split mode is
 // on (FP64, unbatched), else the MFMA GEMM.
 template <typename T>

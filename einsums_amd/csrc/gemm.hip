@@ -201,24 +201,7 @@ __global__ __launch_bounds__(256) void gemm_streamk_fixup(GemmProblem<T> P) {
     int const e0      = int(blockIdx.x) * 256 + int(threadIdx.x);
     int const stride  = int(gridDim.x) * 256;
     T sum[FIXUP_EPT];
-#pragma unroll
-    for (int x = 0; x < FIXUP_EPT; ++x) sum[x] = T(0);
-    if (sk.ksplit) { // split-K: the pieces of tile t in chunk order
-        for (uint64_t c = 0; c < sk.ksplit; ++c) {
-            T const *__restrict__ pc = P.partial + (c * sk.tiles + t) * (BM * BN);
-#pragma unroll
-            for (int x = 0; x < FIXUP_EPT; ++x) sum[x] += pc[e0 + x * stride];
-        }
-    } else {
-        uint64_t g0, g1;
-        sk_owners(sk, t, g0, g1);
-        if (g0 == g1) return;
-        for (uint64_t g = g0; g <= g1; ++g) {
-            T const *__restrict__ pc = P.partial + sk_slot(sk, g, t) * (BM * BN);
-#pragma unroll
-            for (int x = 0; x < FIXUP_EPT; ++x) sum[x] += pc[e0 + x * stride];
-        }
-    }
+    if (!sk_sum_pieces<T, BM * BN>(sk, P.partial, t, e0, stride, sum)) return;
     uint32_t const tiles_mn = P.tiles_m * P.tiles_n;
     int64_t const batch     = int64_t(t / tiles_mn);
     uint32_t tm, tn;
@@ -320,7 +303,7 @@ int launch_dense(GemmProblem<T> &P, int blocks_per_cu, hipStream_t stream, size_
     }
     void *args[] = {&P};
     EIN_HIP_CHECK(hipLaunchKernel(kern, dim3(P.sk.grid), dim3(GEMM_THREADS), args, 0, stream));
-    if (P.sk.units != 0) {
+    if (sk_cuts(P.sk)) {
         gemm_streamk_fixup<T, BM, BN><<<sk_fixup_grid(P.sk, BM * BN), 256, 0, stream>>>(P);
         EIN_LAUNCH_CHECK();
     }
@@ -376,7 +359,7 @@ constexpr CostModel FP32_COST = {{{128, 128, 2, 1.153, 1.018}, {128, 64, 3, 0.60
                                  4.1, 4.8, 0.208, 0.059, 0.300};
 
 double cost_us(CostModel const &M, GemmConfig const &c, int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes,
-               int unaligned) {
+               int unaligned, double slower = 1.0) {
     for (TileCost const &t : M.tiles) {
         if (t.bm != c.bm || t.bn != c.bn) continue;
         uint64_t const cus   = uint64_t(num_cus());
@@ -389,8 +372,10 @@ double cost_us(CostModel const &M, GemmConfig const &c, int64_t m, int64_t n, in
         double const w       = double(work) * t.work * (1 + M.work_unaligned * unaligned);
         double const h       = double(chain) * t.chain * (1 + M.chain_unaligned * unaligned);
         double const w2 = w * w, h2 = h * h;
-        double us = M.launch + std::sqrt(std::sqrt(w2 * w2 + h2 * h2));
-        if (sk.units != 0) us += M.fixup + M.fixup_mb * 1e-6 * double(sk_piece_slots(sk)) * t.bm * t.bn * elem_bytes;
+        double us = M.launch + slower * std::sqrt(std::sqrt(w2 * w2 + h2 * h2));
+        if (sk_cuts(sk)) // and a chain of loads over the pieces of one tile
+            us += M.fixup + M.fixup_mb * 1e-6 * double(sk_piece_slots(sk)) * t.bm * t.bn * elem_bytes +
+                  0.15 * double(slabs) / double(sk.units);
         return us;
     }
     return 0; // not a tile of the model
@@ -424,6 +409,16 @@ GemmConfig refine_gemm_config(GemmConfig const &cfg, int64_t m, int64_t n, int64
     return out;
 }
 } // namespace
+
+double gemm_time_us(int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes, GemmConfig const &cfg, double slower) {
+    return cost_us(elem_bytes == 8 ? FP64_COST : FP32_COST, cfg, m, n, k, batch, elem_bytes, 0, slower);
+}
+
+double gemm_time_us(int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes, bool krow_both, int unaligned) {
+    GemmConfig const cfg = refine_gemm_config(choose_gemm_config(m, n, k, batch, elem_bytes), m, n, k, batch, elem_bytes,
+                                              krow_both, unaligned);
+    return cost_us(elem_bytes == 8 ? FP64_COST : FP32_COST, cfg, m, n, k, batch, elem_bytes, unaligned);
+}
 
 // ------------------------------------------------------------- tuning table
 // Measured GEMM configurations, keyed by the normalised problem (C's unit-stride direction

@@ -32,6 +32,13 @@ struct GemmConfig {
 
 GemmConfig choose_gemm_config(int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes);
 
+// Estimated microseconds of a dense product of 64- or 128-row tiles: with the given
+// configuration and its slabs `slower` than the dense kernel's, or with the configuration that
+// a call takes (`unaligned` operands staged through registers, krow_both: both contiguous
+// along k).
+double gemm_time_us(int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes, GemmConfig const &cfg, double slower);
+double gemm_time_us(int64_t m, int64_t n, int64_t k, int64_t batch, int elem_bytes, bool krow_both, int unaligned);
+
 // Strided (optionally batched) GEMM; `force` overrides the tile heuristic (autotuner).
 template <typename T>
 int gemm_strided(GemmProblem<T> P, GemmConfig const *force, hipStream_t stream);

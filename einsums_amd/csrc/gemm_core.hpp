@@ -244,6 +244,44 @@ inline dim3 sk_fixup_grid(StreamK const &sk, int tile_elems) {
     return dim3(uint32_t(tile_elems / (256 * FIXUP_EPT)), sk.tiles - sk.dp_tiles, 1);
 }
 
+// Sums the pieces of tile t in workgroup (split-K: chunk) order into sum: elements e0 + x * stride
+// of each piece of TILE elements. Returns false for a tile that was finished in place. Four
+// pieces' loads are in flight at once: a tile cut into many (one tile left over by the whole
+// rounds is shared by every CU) is otherwise a chain of load latencies (1176 x 1720 x 1376 FP64,
+// 513 tiles of 64 x 64, the last in 86 pieces: 158 -> 135 us for the product).
+template <typename T, int TILE>
+__device__ __forceinline__ bool sk_sum_pieces(StreamK const &sk, T const *__restrict__ partial, uint64_t t, int e0,
+                                              int stride, T (&sum)[FIXUP_EPT]) {
+    uint64_t g0 = 0, g1 = sk.ksplit - 1;
+    if (!sk.ksplit) {
+        sk_owners(sk, t, g0, g1);
+        if (g0 == g1) return false;
+    }
+#pragma unroll
+    for (int x = 0; x < FIXUP_EPT; ++x) sum[x] = T(0);
+    constexpr int PB = 4;
+    for (uint64_t g = g0; g <= g1; g += PB) {
+        T v[PB][FIXUP_EPT];
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+            if (g + u > g1) continue;
+            T const *pc = partial + (sk.ksplit ? (g + u) * sk.tiles + t : sk_slot(sk, g + u, t)) * TILE;
+#pragma unroll
+            for (int x = 0; x < FIXUP_EPT; ++x) v[u][x] = pc[e0 + x * stride];
+        }
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+            if (g + u > g1) continue;
+#pragma unroll
+            for (int x = 0; x < FIXUP_EPT; ++x) sum[x] += v[u][x];
+        }
+    }
+    return true;
+}
+
+// Whether a schedule cuts any tile (whole tiles per workgroup leave nothing to fix up).
+inline bool sk_cuts(StreamK const &sk) { return sk.units != 0 && (sk.ksplit != 0 || sk.units % sk.slabs != 0); }
+
 // Number of piece slots a launch needs.
 inline uint64_t sk_piece_slots(StreamK const &sk) {
     return sk.ksplit ? uint64_t(sk.grid) : sk.units ? 2ull * (sk.grid - sk.dp_tiles) : 0;

@@ -298,9 +298,9 @@ int launch_wave_tiles(WaveLaunch<T> &P, hipStream_t stream) {
 // the operands' reuse that a wave lacks (FP64 640^3 NT 24 us, here 38; 768^3 33, here 67), and
 // above 32768 steps its split over the whole chip beats 16 waves to a tile (16 x 16 x 100000
 // 352 us, here 519; 64 x 64 x 32768 388, here 175).
-inline bool wave_small(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t max_tiles) {
+inline bool wave_small(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t max_tiles, double max_flops = 4e8) {
     return k <= 32768 && ceil_div(m, 64) * ceil_div(n, 64) <= max_tiles / batch &&
-           2.0 * double(m) * double(n) * double(k) * double(batch) <= 4e8;
+           2.0 * double(m) * double(n) * double(k) * double(batch) <= max_flops;
 }
 
 // Whether the wave kernel can index a problem at all.
