@@ -8,7 +8,7 @@ map from tile coordinates to tiles; absent tiles are zero.
 Their einsums follow BlockAlgebra.hpp:23-52 (block i of C from block i of A and B) and
 TileAlgebra.hpp:18-93 (C scaled once, then every tile triple of the tile grid accumulates
 with prefactor 1). Instead of one library call per block, all the per-block contractions
-become one ``GroupedEinsum`` -- a plan executed as persistent grouped launches -- that can be
+become one ``GroupedEinsum`` -- a plan executed as grouped launches -- that can be
 replayed and captured into a hipGraph.
 """
 from __future__ import annotations
