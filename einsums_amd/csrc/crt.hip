@@ -32,10 +32,7 @@
 // whole cache lines. Row-major planes gave it sixteen halves, and at the same bytes twice the
 // requests (4096^3, 12 moduli: 1378 -> 1259 us from this alone).
 #include <algorithm>
-#include <array>
 #include <cmath>
-#include <map>
-#include <mutex>
 #include <string>
 
 #include "ozaki.hpp"
@@ -551,47 +548,14 @@ int crt_residues(SliceSrc const &S, CrtMods const &K, int32_t *e, int8_t *out, i
     return EIN_SUCCESS;
 }
 
-// The side stream of the current device (created once, default priority) and four events
-// of this host thread on it.
-struct CrtSide {
-    hipStream_t aux = nullptr;
-    hipEvent_t gemm_done[2]  = {nullptr, nullptr};
-    hipEvent_t recon_done[2] = {nullptr, nullptr};
-};
-
-int crt_side(CrtSide &out) {
-    int dev = 0;
-    EIN_HIP_CHECK(hipGetDevice(&dev));
-    {
-        static std::mutex mu;
-        static std::map<int, hipStream_t> aux;
-        std::lock_guard<std::mutex> lock(mu);
-        auto it = aux.find(dev);
-        if (it == aux.end()) {
-            hipStream_t s = nullptr;
-            EIN_HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-            it = aux.emplace(dev, s).first;
-        }
-        out.aux = it->second;
-    }
-    thread_local std::map<int, std::array<hipEvent_t, 4>> events;
-    auto it = events.find(dev);
-    if (it == events.end()) {
-        std::array<hipEvent_t, 4> e{};
-        for (auto &x : e) EIN_HIP_CHECK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
-        it = events.emplace(dev, e).first;
-    }
-    out.gemm_done[0]  = it->second[0];
-    out.gemm_done[1]  = it->second[1];
-    out.recon_done[0] = it->second[2];
-    out.recon_done[1] = it->second[3];
-    return EIN_SUCCESS;
-}
-
 } // namespace
 
-// Residue planes are written for column panels of at most this many bytes.
-constexpr size_t CRT_PANEL_BYTES = size_t(8) << 30;
+// Residue planes are written for column panels of at most this many bytes, each reconstructed
+// before the next is formed. On a side stream, beside the next panel's residue GEMM, the
+// reconstruction takes CUs from workgroups that each own a fixed share of the panel:
+// 65536^2 x 2304 (12 moduli) 174.8 ms, in order 142.3; 49152^2 93.7 and 79.2; panels of 8 GiB
+// 142.5 and 79.9.
+constexpr size_t CRT_PANEL_BYTES = size_t(4) << 30;
 
 int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
     if (nmod < CRT_MIN_MODULI || nmod > CRT_MAX_MODS)
@@ -606,18 +570,9 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
 
     uint32_t const tiles_m = uint32_t(ceil_div(P.m, CG_TI));
     int64_t const ldr      = int64_t(tiles_m) * CG_TI;
-    // column panels of whole 256-column tiles whose residue planes take at most
-    // CRT_PANEL_BYTES; with more than one panel, two plane buffers of half that so the
-    // reconstruction of panel p (HBM-bound) runs on a side stream while the residue GEMM of
-    // panel p+1 (MFMA-bound) runs on the caller's stream
-    auto panel_cols = [&](size_t budget) {
-        int64_t c = int64_t(budget / (size_t(nmod) * size_t(ldr))) / CG_TI * CG_TI;
-        return std::max<int64_t>(CG_TI, std::min<int64_t>(c, ceil_div(P.n, CG_TI) * CG_TI));
-    };
-    int64_t pn      = panel_cols(CRT_PANEL_BYTES);
-    bool const fork = pn < P.n && !stream_capturing(stream);
-    if (fork) pn = panel_cols(CRT_PANEL_BYTES / 2);
-    int const nbuf = fork ? 2 : 1;
+    // column panels of whole 256-column tiles whose residue planes take at most CRT_PANEL_BYTES
+    int64_t pn = int64_t(CRT_PANEL_BYTES / (size_t(nmod) * size_t(ldr))) / CG_TI * CG_TI;
+    pn         = std::max<int64_t>(CG_TI, std::min<int64_t>(pn, ceil_div(P.n, CG_TI) * CG_TI));
 
     int64_t const a_plane = ceil_div(P.m, 16) * 16 * kp, b_plane = ceil_div(P.n, 16) * 16 * kp;
     size_t const a_bytes = size_t(nmod) * size_t(a_plane);
@@ -626,7 +581,7 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
     auto up              = [](size_t x) { return (x + 255) / 256 * 256; };
     size_t const b_off   = up(a_bytes);
     size_t const r_off   = b_off + up(b_bytes);
-    size_t const ea_off  = r_off + size_t(nbuf) * up(r_bytes);
+    size_t const ea_off  = r_off + up(r_bytes);
     size_t const eb_off  = ea_off + up(size_t(P.m) * 4);
     size_t const x_off   = eb_off + up(size_t(P.n) * 4);
     // the GEMM's tiles read up to CG_TI rows past the last plane of an operand
@@ -647,80 +602,57 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
     EIN_TRY(crt_residues(SA, K, ea, As, a_plane, scratch, stream));
     EIN_TRY(crt_residues(SB, K, eb, Bs, b_plane, scratch, stream));
 
-    CrtSide side;
-    if (fork) EIN_TRY(crt_side(side));
-    int last    = -1; // plane buffer of the last reconstruction queued on the side stream
-    auto panels = [&]() -> int {
-        for (int64_t j0 = 0, panel = 0; j0 < P.n; j0 += pn, ++panel) {
-            int64_t const nj = std::min(pn, P.n - j0);
-            int const b      = fork ? int(panel & 1) : 0;
-            uint8_t *Rb      = R + size_t(b) * up(r_bytes);
-            if (fork && panel >= 2) EIN_HIP_CHECK(hipStreamWaitEvent(stream, side.recon_done[b], 0)); // buffer b free
-            CrtGemm G{};
-            G.m       = P.m;
-            G.n       = nj;
-            G.kp      = kp;
-            G.a_plane = a_plane;
-            G.b_plane = b_plane;
-            G.A       = As;
-            G.B       = Bs + j0 * kp;
-            G.R       = Rb;
-            G.ldr     = ldr;
-            G.r_plane = nj * ldr;
-            G.tiles_m = tiles_m;
-            G.tiles_n = uint32_t(ceil_div(nj, CG_TJ));
-            G.K       = K;
-            uint64_t const grid = uint64_t(G.tiles_m) * G.tiles_n * uint64_t(nmod);
-            if (grid > 0x7fffffffu) return fail(EIN_ERROR_UNSUPPORTED, "split gemm: tile grid too large");
-            for (int64_t k0 = 0; k0 < kp; k0 += int64_t(CRT_FOLD_STAGES) * CG_KS) {
-                G.k0         = k0;
-                G.kc         = std::min<int64_t>(int64_t(CRT_FOLD_STAGES) * CG_KS, kp - k0);
-                G.accumulate = k0 > 0;
-                G.items = uint32_t(grid);
-                crt_gemm_kernel<<<uint32_t(std::min<uint64_t>(grid, 2 * uint64_t(num_cus()))), 64 * CG_WAVES, 0, stream>>>(
-                    G);
-                EIN_LAUNCH_CHECK();
-            }
-
-            hipStream_t rs = stream;
-            if (fork) {
-                EIN_HIP_CHECK(hipEventRecord(side.gemm_done[b], stream));
-                EIN_HIP_CHECK(hipStreamWaitEvent(side.aux, side.gemm_done[b], 0));
-                rs = side.aux;
-            }
-            CrtRec Q{};
-            Q.m       = P.m;
-            Q.n       = nj;
-            Q.R       = Rb;
-            Q.ldr     = ldr;
-            Q.r_plane = nj * ldr;
-            Q.ea      = ea;
-            Q.eb      = eb + j0;
-            Q.C       = P.C + j0 * P.c_sn;
-            Q.c_sm    = P.c_sm;
-            Q.c_sn    = P.c_sn;
-            Q.alpha   = P.alpha;
-            Q.beta    = P.beta;
-            Q.W       = W;
-            int64_t const threads = nj * (ldr / 4);
-            if (ceil_div(threads, 256) > 0x7fffffff) return fail(EIN_ERROR_UNSUPPORTED, "split gemm: panel too large");
-            bool const vec = Q.c_sm == 1 && Q.c_sn % 2 == 0 && reinterpret_cast<uintptr_t>(Q.C) % 16 == 0;
-            auto const rec = crt_limbs(nmod) == 3 ? (vec ? crt_reconstruct_kernel<3, true> : crt_reconstruct_kernel<3, false>)
-                                                  : (vec ? crt_reconstruct_kernel<4, true> : crt_reconstruct_kernel<4, false>);
-            rec<<<uint32_t(ceil_div(threads, 256)), 256, 0, rs>>>(Q);
-            if (fork) {
-                last = b;
-                EIN_HIP_CHECK(hipEventRecord(side.recon_done[b], side.aux));
-            }
+    for (int64_t j0 = 0; j0 < P.n; j0 += pn) {
+        int64_t const nj = std::min(pn, P.n - j0);
+        CrtGemm G{};
+        G.m       = P.m;
+        G.n       = nj;
+        G.kp      = kp;
+        G.a_plane = a_plane;
+        G.b_plane = b_plane;
+        G.A       = As;
+        G.B       = Bs + j0 * kp;
+        G.R       = R;
+        G.ldr     = ldr;
+        G.r_plane = nj * ldr;
+        G.tiles_m = tiles_m;
+        G.tiles_n = uint32_t(ceil_div(nj, CG_TJ));
+        G.K       = K;
+        uint64_t const grid = uint64_t(G.tiles_m) * G.tiles_n * uint64_t(nmod);
+        if (grid > 0x7fffffffu) return fail(EIN_ERROR_UNSUPPORTED, "split gemm: tile grid too large");
+        for (int64_t k0 = 0; k0 < kp; k0 += int64_t(CRT_FOLD_STAGES) * CG_KS) {
+            G.k0         = k0;
+            G.kc         = std::min<int64_t>(int64_t(CRT_FOLD_STAGES) * CG_KS, kp - k0);
+            G.accumulate = k0 > 0;
+            G.items      = uint32_t(grid);
+            crt_gemm_kernel<<<uint32_t(std::min<uint64_t>(grid, 2 * uint64_t(num_cus()))), 64 * CG_WAVES, 0, stream>>>(
+                G);
             EIN_LAUNCH_CHECK();
         }
-        return EIN_SUCCESS;
-    };
-    int const status = panels();
-    // join, also after a failure, so no queued reconstruction outlives the call's workspace:
-    // the side stream runs the reconstructions in order, so the last one covers all
-    if (last >= 0) EIN_HIP_CHECK(hipStreamWaitEvent(stream, side.recon_done[last], 0));
-    return status;
+
+        CrtRec Q{};
+        Q.m       = P.m;
+        Q.n       = nj;
+        Q.R       = R;
+        Q.ldr     = ldr;
+        Q.r_plane = nj * ldr;
+        Q.ea      = ea;
+        Q.eb      = eb + j0;
+        Q.C       = P.C + j0 * P.c_sn;
+        Q.c_sm    = P.c_sm;
+        Q.c_sn    = P.c_sn;
+        Q.alpha   = P.alpha;
+        Q.beta    = P.beta;
+        Q.W       = W;
+        int64_t const threads = nj * (ldr / 4);
+        if (ceil_div(threads, 256) > 0x7fffffff) return fail(EIN_ERROR_UNSUPPORTED, "split gemm: panel too large");
+        bool const vec = Q.c_sm == 1 && Q.c_sn % 2 == 0 && reinterpret_cast<uintptr_t>(Q.C) % 16 == 0;
+        auto const rec = crt_limbs(nmod) == 3 ? (vec ? crt_reconstruct_kernel<3, true> : crt_reconstruct_kernel<3, false>)
+                                              : (vec ? crt_reconstruct_kernel<4, true> : crt_reconstruct_kernel<4, false>);
+        rec<<<uint32_t(ceil_div(threads, 256)), 256, 0, stream>>>(Q);
+        EIN_LAUNCH_CHECK();
+    }
+    return EIN_SUCCESS;
 }
 
 int crt_bits(int nmod, int64_t k) {

@@ -1,4 +1,4 @@
-// Block-sparse device tensors and their einsums as grouped persistent launches.
+// Block-sparse device tensors and their einsums as grouped launches.
 //
 // Reference types mirrored: BlockDeviceTensor (libs/Einsums/Tensor/include/Einsums/Tensor/
 // BlockTensor.hpp:46,119-131: hypercubic blocks, one extent per block) and
@@ -6,7 +6,7 @@
 // coordinates to tiles, absent tiles are zero). einsum on them follows BlockAlgebra.hpp:23-52
 // (block i from blocks i) and TileAlgebra.hpp:18-93 (C scaled once, then every tile triple of
 // the tile grid accumulates with prefactor 1); all block contractions of one call are handed
-// to the backend as one grouped plan (ein_grouped_plan_*), i.e. persistent launches instead of
+// to the backend as one grouped plan (ein_grouped_plan_*), i.e. a few launches instead of
 // one library call per block.
 #pragma once
 

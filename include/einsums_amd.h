@@ -147,8 +147,9 @@ int ein_axpby_f32(int64_t n, float alpha, const float *x, int64_t incx, float be
  * GEMM-mapped einsum looks its problem up in a process-wide table keyed by the normalised
  * problem (element size, m, n, k, batch, whether A and B are contiguous along k); an entry
  * overrides the built-in tile heuristic. With tuning mode on, a GEMM whose key is absent
- * first times every candidate (tile 128/64 x 128/64; hybrid stream-K, data-parallel or
- * split-K over XCD-local contraction chunks; planned workgroups per CU) on its own
+ * first times every candidate (tile 128/64 x 128/64, 96 x 96, FP32 256 x 128; hybrid stream-K,
+ * data-parallel or split-K over XCD-local contraction chunks; planned workgroups per CU; for
+ * small products one wave per tile, written 16 x 16) on its own
  * operands, writing a scratch C, and stores the
  * fastest (not while its stream is captured). No counterpart in the reference (its GEMMs
  * are vendor BLAS calls). The table is saved and loaded as text.
@@ -299,7 +300,7 @@ int ein_einsum_adjoint_f32(int32_t wrt, float alpha, const ein_tensor_desc *C, c
                            float *g, int32_t *algorithm_used, ein_stream_t stream);
 
 /* Grouped contractions: many independent generic contractions (blocks of a block-sparse
- * einsum, batches of uneven GEMMs) planned once and run as persistent launches -- one per
+ * einsum, batches of uneven GEMMs) planned once and run as grouped launches -- one set per
  * wave of items whose outputs differ (items writing the same C pointer go to later waves,
  * in list order). Plan creation copies descriptors to device memory (synchronous);
  * execution is launches only, so it can be captured into a hipGraph. The autotuner times
@@ -345,7 +346,8 @@ int ein_einsum_execute_f32(int32_t algorithm, float c_prefactor, const ein_tenso
  * (libs/Einsums/BLAS/include/Einsums/BLAS.hpp:306; linear_algebra::syev, LinearAlgebra.hpp:362).
  * Column-major; uplo names the triangle read; job 'V' overwrites A with orthonormal
  * eigenvectors (columns), 'N' leaves A; W gets the eigenvalues ascending. Cyclic Jacobi,
- * n <= 1024; *info = 1 if 60 sweeps do not converge. Workspace 2*n*n elements from the pool. */
+ * n <= 1024; *info = 1 if 60 sweeps do not converge. Workspace below 2*n*n elements, none to
+ * n = 114 (FP64). */
 int ein_syev_f64(char job, char uplo, int64_t n, double *A, int64_t lda, double *W, int32_t *info, ein_stream_t stream);
 int ein_syev_f32(char job, char uplo, int64_t n, float *A, int64_t lda, float *W, int32_t *info, ein_stream_t stream);
 /* gesv replaces blas::gesv(n, nrhs, a, lda, ipiv, b, ldb) (BLAS.hpp:529; linear_algebra::gesv,
