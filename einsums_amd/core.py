@@ -452,21 +452,22 @@ def _syev_body(A, W, compute_vectors, check_info):
         raise DimensionError("syev: W must have n entries")
     if W.dtype != A.dtype or not W.is_contiguous():
         raise TypeError("syev: W must be a contiguous vector of A's dtype")
-    info = torch.empty((), dtype=torch.int32, device=A.device)  # the solver writes it, whatever n
-    job = b"V" if compute_vectors else b"N"
-    fn = _fn("ein_syev", A.dtype)
-    if A.stride(0) == 1 and A.stride(1) >= max(1, n):
-        # column-major storage: the upper triangle as the solver sees it
-        check(fn(job, b"U", n, _ptr(A), A.stride(1), _ptr(W), _ptr(info), stream_handle(stream)), "syev")
-    elif A.stride(1) == 1 and A.stride(0) >= max(1, n):
-        # row-major storage is the column-major transpose: its upper triangle is the solver's
-        # lower one, and the eigenvector columns come out as rows
-        check(fn(job, b"L", n, _ptr(A), A.stride(0), _ptr(W), _ptr(info), stream_handle(stream)), "syev")
-        if compute_vectors:
+    columns = A.stride(0) == 1 and A.stride(1) >= max(1, n)
+    rows = A.stride(1) == 1 and A.stride(0) >= max(1, n)
+    if columns or rows:
+        info = torch.empty((), dtype=torch.int32, device=A.device)  # the solver writes it, whatever n
+        # column-major storage: the upper triangle as the solver sees it. Row-major storage is the
+        # column-major transpose: its upper triangle is the solver's lower one, and the
+        # eigenvector columns come out as rows
+        check(_fn("ein_syev", A.dtype)(b"V" if compute_vectors else b"N", b"U" if columns else b"L", n, _ptr(A),
+                                       A.stride(1) if columns else A.stride(0), _ptr(W), _ptr(info),
+                                       stream_handle(stream)), "syev")
+        if compute_vectors and not columns:
             A.copy_(A.t().contiguous())
     else:
-        tmp = A.contiguous()
-        syev(tmp, W, compute_vectors, stream, check_info=False)
+        # on a copy in rows (a 1 x 1 view counts as contiguous with any strides); its status is ours
+        tmp = A.clone(memory_format=torch.contiguous_format)
+        info = _syev_body(tmp, W, compute_vectors, check_info=False)
         A.copy_(tmp)
     if check_info and int(info.item()) != 0:
         raise EinsumsError("syev: the Jacobi iteration did not converge")
