@@ -191,11 +191,11 @@ __global__ __launch_bounds__(256) void fock_jk16_kernel(int n, double const *__r
 // or K reduction comes between two slabs of the same a. MR = ceil(n / 16) rows c = wave + 16 i;
 // VEC: a lane reads d = 2l, 2l+1 as 16 bytes (even n, 16-byte aligned rows), otherwise d = l
 // and l + 64. All loads are unconditional, from clamped addresses, so that the wait before a
-// slab counts exactly the loads behind it; what lies outside is dropped where it is summed.
+// slab counts exactly the loads behind it; what lies outside is dropped before it is summed.
 // J(a,b) sums its waves from LDS at the end; K is written per a as piece 2w (the first a of
 // workgroup w) or 2w+1. One workgroup per slab, whose shuffle reductions and start nothing
 // overlapped, took 195 + 13.5 us at n = 96 (3.4 TB/s over the call). Now, per call: n = 65 47 us
-// (before 77), 96 126 us = 5.4 TB/s (202), 97 161 (314), 112 215 (435), 127 425 (620), 128 362 (621).
+// (before 77), 96 126 us = 5.4 TB/s (202), 97 146 (314), 112 215 (435), 127 367 (620), 128 361 (621).
 constexpr int FOCK_WAVES = 16, FOCK_UNITS = 64; // LDS for the J sums of 64 slabs
 
 template <int MR, bool VEC>
@@ -211,9 +211,9 @@ __global__ __launch_bounds__(64 * FOCK_WAVES) void fock_jk_stream_kernel(int n, 
     int const wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     int const lane = int(threadIdx.x) & 63;
     int const nn   = n * n;
-    if constexpr (D_LDS) {
-        for (int c = wave; c < n; c += FOCK_WAVES)
-            for (int d = lane; d < n; d += 64) dl[c * n + d] = D[int64_t(c) * ldd + d];
+    if constexpr (D_LDS) { // zeros outside
+        for (int c = wave; c < FOCK_WAVES * MR; c += FOCK_WAVES)
+            for (int d = lane; d < FOCK_MAX_N; d += 64) dl[c * FOCK_MAX_N + d] = c < n && d < n ? D[int64_t(c) * ldd + d] : 0.0;
         __syncthreads();
     }
     int const s0 = int(blockIdx.x) * units, s1 = s0 + units < nn ? s0 + units : nn;
@@ -227,8 +227,12 @@ __global__ __launch_bounds__(64 * FOCK_WAVES) void fock_jk_stream_kernel(int n, 
             v[0] = t.x;
             v[1] = t.y;
         } else {
-            v[0] = row[d0];
-            v[1] = row[d1];
+            // byte offsets without a sign, opaque at each load, which then adds them to the row's
+            // address by itself: the compiler would keep a 64-bit address per row, and spill
+            uint32_t o0 = 8u * uint32_t(d0), o1 = 8u * uint32_t(d1);
+            asm volatile("" : "+v"(o0), "+v"(o1));
+            v[0] = *reinterpret_cast<double const *>(reinterpret_cast<char const *>(row) + o0);
+            v[1] = *reinterpret_cast<double const *>(reinterpret_cast<char const *>(row) + o1);
         }
     };
     int row[MR]; // offset of the wave's rows in a slab
@@ -261,15 +265,20 @@ __global__ __launch_bounds__(64 * FOCK_WAVES) void fock_jk_stream_kernel(int n, 
     };
     auto work = [&](int s, double (&x)[MR][2], double (&db)[2]) {
         double jsum = 0.0;
-        int e0 = d0, e1 = d1;
-        if constexpr (D_LDS) asm volatile("" : "+v"(e0), "+v"(e1)); // read each time, not kept in registers
+        double const dby = in1 ? db[1] : 0.0;
+        int e0 = wave * FOCK_MAX_N + d0;
+        if constexpr (D_LDS) asm volatile("" : "+v"(e0)); // read each time, not kept in registers
+        int const e1 = VEC ? e0 + 1 : e0 + 64;
 #pragma unroll
         for (int i = 0; i < MR; ++i) {
-            double const y = in1 ? x[i][1] : 0.0;
-            double const j = x[i][0] * (D_LDS ? dl[row[i] + e0] : dc[D_LDS ? 0 : i][0]) +
-                             y * (D_LDS ? dl[row[i] + e1] : dc[D_LDS ? 0 : i][1]);
+            // a lane without a second element has zeros on both sides of its products: what its
+            // clamped address holds may be an infinity, in g as in D
+            constexpr int ROW = FOCK_WAVES * FOCK_MAX_N;
+            double const y    = in1 ? x[i][1] : 0.0;
+            double const j    = x[i][0] * (D_LDS ? dl[e0 + i * ROW] : dc[D_LDS ? 0 : i][0]) +
+                             y * (D_LDS ? dl[e1 + i * ROW] : dc[D_LDS ? 0 : i][1]);
             jsum += i < MR - 1 || last_in ? j : 0.0;
-            kacc[i] += x[i][0] * db[0] + y * db[1];
+            kacc[i] += x[i][0] * db[0] + y * dby;
         }
         jsum = wave_reduce_sum(in0 ? jsum : 0.0);
         if (lane == 0) jred[s - s0][wave] = jsum;
