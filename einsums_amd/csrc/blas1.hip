@@ -483,15 +483,18 @@ int ger_impl(int64_t m, int64_t n, T alpha, T const *x, int64_t incx, T const *y
     int64_t const r  = vec ? m / VW : m; // threads along the rows
     int tr           = 0;
     while (tr < 8 && (int64_t{1} << tr) < r) ++tr;
-    int64_t const rb = ceil_div(r, int64_t{1} << tr);
     int64_t const cb = std::min<int64_t>(ceil_div(n, int64_t(256 >> tr) * GER_COLS), 65535);
-    if (rb > 0x7fffffff) return fail(EIN_ERROR_UNSUPPORTED, "ger: more than 2^39 rows");
-    dim3 const grid{uint32_t(rb), uint32_t(cb)};
-    if (vec)
-        ger_kernel<T, VW><<<grid, 256, 0, stream>>>(m, n, alpha, x, incx, y, incy, beta, A, rs, lda, tr);
-    else
-        ger_kernel<T, 1><<<grid, 256, 0, stream>>>(m, n, alpha, x, incx, y, incy, beta, A, rs, lda, tr);
-    EIN_LAUNCH_CHECK();
+    // rows of one launch: a grid holds fewer than 2^32 threads (and is cut without an error beyond)
+    int64_t const rows = int64_t((1 << 24) - 1) * (int64_t{1} << tr) * (vec ? VW : 1);
+    for (int64_t i0 = 0; i0 < m; i0 += rows) {
+        int64_t const mi = std::min(rows, m - i0);
+        dim3 const grid{uint32_t(ceil_div(vec ? mi / VW : mi, int64_t{1} << tr)), uint32_t(cb)};
+        if (vec)
+            ger_kernel<T, VW><<<grid, 256, 0, stream>>>(mi, n, alpha, x + i0 * incx, incx, y, incy, beta, A + i0 * rs, rs, lda, tr);
+        else
+            ger_kernel<T, 1><<<grid, 256, 0, stream>>>(mi, n, alpha, x + i0 * incx, incx, y, incy, beta, A + i0 * rs, rs, lda, tr);
+        EIN_LAUNCH_CHECK();
+    }
     return EIN_SUCCESS;
 }
 
