@@ -1504,14 +1504,17 @@ int plan_launch(GroupedPlan const &plan, int bm_index, hipStream_t stream) {
             EIN_TRY(tensor_scale<T>(ps.C, static_cast<T *>(ps.c), T(ps.factor), stream));
         uint32_t const nt = w.ntiles[bm_index];
         if (nt != 0) {
-            uint32_t const grid = uint32_t(ceil_div(nt, 4));
             auto const *items   = static_cast<WaveItem<T> const *>(w.d_items);
             auto const *tiles   = static_cast<WaveTile const *>(w.d_tiles[bm_index]);
-            if (bm_index == 1)
-                grouped_wave_kernel<T, 4><<<grid, GEMM_THREADS, 0, stream>>>(items, tiles, nt);
-            else
-                grouped_wave_kernel<T, 2><<<grid, GEMM_THREADS, 0, stream>>>(items, tiles, nt);
-            EIN_LAUNCH_CHECK();
+            EIN_TRY(for_wave_parts(nt, [&](uint32_t first, uint32_t count) {
+                uint32_t const grid = uint32_t(ceil_div(count, 4));
+                if (bm_index == 1)
+                    grouped_wave_kernel<T, 4><<<grid, GEMM_THREADS, 0, stream>>>(items, tiles + first, count);
+                else
+                    grouped_wave_kernel<T, 2><<<grid, GEMM_THREADS, 0, stream>>>(items, tiles + first, count);
+                EIN_LAUNCH_CHECK();
+                return EIN_SUCCESS;
+            }));
         }
         for (auto const &it : w.large)
             EIN_TRY(einsum_execute<T>(EIN_ALG_INDETERMINATE, T(it.c_prefactor), it.C, static_cast<T *>(it.c),

@@ -223,6 +223,7 @@ struct WaveLaunch {
     int64_t a_sb, b_sb, c_sb;  // batch strides of a dense GEMM
     int64_t batch;
     uint32_t tiles_m, tiles_n, ntiles;
+    uint32_t first; // tile of the launch's first wave
 };
 
 template <typename T>
@@ -255,7 +256,7 @@ struct DenseOffsets {
 template <typename T, int FM, int FN, int KS, bool DENSE>
 __global__ __launch_bounds__(KS == 1 ? GEMM_THREADS : 64 * KS, KS > 4 ? 1 : 2) void wave_kernel(WaveLaunch<T> P) {
     int const w      = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint32_t const t = KS == 1 ? blockIdx.x * 4 + w : blockIdx.x;
+    uint32_t const t = KS == 1 ? P.first + blockIdx.x * 4 + w : blockIdx.x;
     if (t >= P.ntiles) return;
     __shared__ T sums[KS == 1 ? 1 : KS * FM * FN * 256];
     uint32_t const mn = P.tiles_m * P.tiles_n;
@@ -279,6 +280,20 @@ __global__ __launch_bounds__(KS == 1 ? GEMM_THREADS : 64 * KS, KS > 4 ? 1 : 2) v
     }
 }
 
+// A grid holds fewer than 2^32 threads (beyond, it is cut without an error), so this many tiles
+// of a wave each, four to a workgroup, are the most of one launch; longer lists go in parts.
+constexpr uint32_t WAVE_TILES_MAX = (1u << 26) - 4;
+
+template <typename F>
+int for_wave_parts(uint32_t ntiles, F const &launch) {
+    for (uint32_t first = 0; first < ntiles;) {
+        uint32_t const count = ntiles - first < WAVE_TILES_MAX ? ntiles - first : WAVE_TILES_MAX;
+        EIN_TRY(launch(first, count));
+        first += count;
+    }
+    return EIN_SUCCESS;
+}
+
 template <typename T, int FM, int FN, int KS, bool DENSE>
 int launch_wave_tiles(WaveLaunch<T> &P, hipStream_t stream) {
     int64_t const tm = ceil_div(P.it.m, 16 * FM), tn = ceil_div(P.it.n, 16 * FN);
@@ -286,10 +301,18 @@ int launch_wave_tiles(WaveLaunch<T> &P, hipStream_t stream) {
     P.tiles_m = uint32_t(tm);
     P.tiles_n = uint32_t(tn);
     P.ntiles  = uint32_t(tm * tn * P.batch);
-    uint32_t const grid = KS == 1 ? uint32_t(ceil_div(P.ntiles, 4)) : P.ntiles;
-    wave_kernel<T, FM, FN, KS, DENSE><<<grid, KS == 1 ? GEMM_THREADS : 64 * KS, 0, stream>>>(P);
-    EIN_LAUNCH_CHECK();
-    return EIN_SUCCESS;
+    if constexpr (KS > 1) { // few tiles (launch_wave)
+        wave_kernel<T, FM, FN, KS, DENSE><<<P.ntiles, 64 * KS, 0, stream>>>(P);
+        EIN_LAUNCH_CHECK();
+        return EIN_SUCCESS;
+    } else {
+        return for_wave_parts(P.ntiles, [&](uint32_t first, uint32_t count) {
+            P.first = first;
+            wave_kernel<T, FM, FN, KS, DENSE><<<uint32_t(ceil_div(count, 4)), GEMM_THREADS, 0, stream>>>(P);
+            EIN_LAUNCH_CHECK();
+            return EIN_SUCCESS;
+        });
+    }
 }
 
 // Whether a problem is small for tiles staged through LDS: fewer of their 64 x 64 tiles than
