@@ -329,7 +329,8 @@ inline bool wave_small(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t m
 // Whether the wave kernel can index a problem at all.
 inline bool wave_fits(int64_t m, int64_t n, int64_t k, int64_t batch) {
     int64_t const most = int64_t{1} << 30;
-    return m < most && n < most && k < most && batch < most && ceil_div(m, 16) * ceil_div(n, 16) < most / batch;
+    auto extent        = [&](int64_t x) { return x > 0 && x < most; };
+    return extent(m) && extent(n) && extent(k) && extent(batch) && ceil_div(m, 16) * ceil_div(n, 16) < most / batch;
 }
 
 // Launches one problem with the largest tiles that still give every SIMD (four per CU) one, and
