@@ -630,11 +630,14 @@ int pack_digits(T const *src, std::vector<std::pair<std::vector<Digit> const *, 
 // into C by the permute. Digit orders are chosen to fold as much as possible. The route
 // is taken (`taken` = true) when nothing is packed, or when packing, dense product and staging
 // are put below gather_us, the estimate of the gather GEMM (0: only if nothing is packed).
-// Fitted to "mbej <- jnfb, mnef" (o 9..32, v 43..104) and "pqrs <- pmrs, mq" (36..100) in FP64 and
-// FP32: over 44 of them the choice loses at most 6% against the better route, where 0.45 of
-// the dense product's time as the line for the extra traffic took the gather for 17 x 51 (FP64 145 us,
-// packed 66), 13 x 77 (207, 92), 20 x 60 (133, 105), 16 x 64 (82, 71).
-constexpr double GATHER_SLOWER[] = {1.65, 1.1}, GATHER_UNALIGNED[] = {1.5, 1.0}; // FP64, FP32
+// FP64 is fitted to "mbej <- jnfb, mnef" (o 9..32, v 43..104) and "pqrs <- pmrs, mq" (36..100): over
+// 22 of them the choice loses at most 6% against the better route, where 0.45 of the dense
+// product's time as the line for the extra traffic took the gather for 17 x 51 (FP64 145 us, packed
+// 66), 13 x 77 (207, 92), 20 x 60 (133, 105), 16 x 64 (82, 71). FP32 is fitted to 290 products, those
+// two and six forms of "acdb <- aebf, fced" with extents 6..56, timed by both routes: it loses 0.06%
+// in the mean and at most 8% (mbej 24, 96: packed 262 us, gathered 320; "pqrs" 64: 99 and 64), and
+// chooses the same up to 1.5 and 1.9. FP64 on 286 products of those kinds: 0.2%, at most 14%.
+constexpr double GATHER_SLOWER[] = {1.65, 1.3}, GATHER_UNALIGNED[] = {1.5, 1.3}; // FP64, FP32
 
 template <typename T>
 int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, std::vector<Digit> const &vn,
@@ -688,7 +691,7 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
             };
             int const ua = unaligned(best.a_ok, best.as, M, a), ub = unaligned(best.b_ok, best.bs, N, b);
             double const dense = gemm_time_us(M, N, K, NB, int(sizeof(T)), true, ua + ub);
-            double const extra = 2e6 * sizeof(T) * best.moved / 5e12 + (sizeof(T) == 8 ? 4.0 : 5.0) * launches;
+            double const extra = 2e6 * sizeof(T) * best.moved / 5e12 + (sizeof(T) == 8 ? 4.0 : 3.0) * launches;
             below              = dense + extra < 0.95 * gather_us;
         }
         if (!below) return EIN_SUCCESS;

@@ -380,7 +380,7 @@ double cost_us(CostModel const &M, GemmConfig const &c, int64_t m, int64_t n, in
                   0.15 * double(slabs) / double(sk.units);
         return us;
     }
-    return 0; // not a tile of the model
+    return HUGE_VAL; // not a tile of the model
 }
 
 // cfg, or a configuration that the model puts at least 6% below it: nearer than that its error
@@ -392,10 +392,11 @@ GemmConfig refine_gemm_config(GemmConfig const &cfg, int64_t m, int64_t n, int64
     CostModel const &M = elem_bytes == 8 ? FP64_COST : FP32_COST;
     double best        = 0.94 * cost_us(M, cfg, m, n, k, batch, elem_bytes, unaligned);
     GemmConfig out     = cfg;
+    if (std::isinf(best)) return cfg; // nothing to compare with
     static constexpr int cands[][4] = {{64, 64, 0, 0},   {64, 64, 0, 1},  {64, 64, 1, 0}, {128, 128, 0, 0},
                                        {128, 128, 0, 1}, {96, 96, 0, 0}, {128, 64, 0, 1}};
     for (auto const &c : cands) {
-        if (c[0] == 96 && !krow_both) continue;
+        if (c[0] == 96 && !(krow_both && elem_bytes == 8)) continue; // as its kernel
         if (c[0] != c[1] && elem_bytes == 8) continue; // FP64: never more than 1% ahead of the others
         GemmConfig g;
         g.bm            = c[0];
