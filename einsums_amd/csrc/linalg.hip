@@ -84,6 +84,41 @@ __host__ __device__ __forceinline__ int tri(int i, int j) {
     return lo + hi * (hi + 1) / 2;
 }
 
+// The convergence norm is a sum of squares, which leaves the range of the type long before the
+// entries do (FP32: near 1e19 and 1e-19). Where `fro`, the sum over the packed triangle M of
+// order m, or n^2 eps^2 times it would, M is scaled so that its largest entry is in [1/2, 1), and
+// `fro` is formed again. Powers of two scale exactly and the rotations do not depend on them;
+// returns the exponent by which the eigenvalues are scaled back. With an infinite entry no scale
+// helps: `fro` stays infinite.
+template <typename T, typename Sum>
+__device__ __forceinline__ int bring_into_range(T *M, int m, T *red, Sum const &sum, T &fro) {
+    constexpr T LEAST = sizeof(T) == 8 ? T(1e-200) : T(1e-20), MOST = sizeof(T) == 8 ? T(1e300) : T(1e37);
+    // the same in every lane; the compiler has to know, or the sweeps' scalar state goes to vectors
+    auto uniform = [](bool x) { return __builtin_amdgcn_readfirstlane(int(x)) != 0; };
+    if (uniform(fro >= LEAST && fro <= MOST)) return 0;
+    int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    T big = T(0);
+    for (int x = threadIdx.x; x < m * (m + 1) / 2; x += blockDim.x) big = fmax(big, fabs(M[x]));
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+    __syncthreads();
+    if (lane == 0) red[wave] = big;
+    __syncthreads();
+    for (int i = 0; i < waves; ++i) big = fmax(big, red[i]);
+    if (uniform(!(big > T(0)) || isinf(big))) return 0;
+    int e;
+    (void)frexp(big, &e);
+    T f = T(0);
+    for (int j = wave; j < m; j += waves)
+        for (int i = lane; i <= j; i += 64) {
+            T const v    = ldexp(M[tri(i, j)], -e);
+            M[tri(i, j)] = v;
+            f += i == j ? v * v : T(2) * v * v;
+        }
+    fro = sum(f);
+    return __builtin_amdgcn_readfirstlane(e);
+}
+
 // Jacobi for n <= 64 with M and V in LDS, on one workgroup. What bounds it is the chain of
 // steps (n-1 per sweep), each waiting for the one before, so the work between its barriers is
 // what is kept short:
@@ -156,8 +191,9 @@ __global__ __launch_bounds__(LA_THREADS) void syev_lds_kernel(int n, int upper, 
             if (vectors && i < n) V[i + position(j) * n] = i == j ? T(1) : T(0);
         }
     fro = sum(fro); // also orders the writes above before the reads below
+    int const back = bring_into_range(lds, m, red, sum, fro);
     T const eps   = sizeof(T) == 8 ? T(2.220446049250313e-16) : T(1.1920929e-7);
-    T const limit = T(n) * T(n) * eps * eps * fro;
+    T const limit = isinf(fro) ? T(0) : T(n) * T(n) * eps * eps * fro;
 
     // the diagonal block of the thread's rotation: where it is read and written
     int const rot  = tid < npairs ? tid : 0;
@@ -279,7 +315,7 @@ __global__ __launch_bounds__(LA_THREADS) void syev_lds_kernel(int n, int upper, 
         }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) pos += __shfl_xor(pos, o, 64);
-        if (lane == 0) W[pos] = d;
+        if (lane == 0) W[pos] = ldexp(d, back);
         if (vectors)
             for (int k = lane; k < n; k += 64) A[k + int64_t(pos) * lda] = V[k + at * n];
     }
@@ -352,8 +388,9 @@ __global__ __launch_bounds__(LA_THREADS) void syev_jacobi_kernel(int n, int uppe
             if (vectors && i < n && j < n) V[i + int64_t(j) * n] = i == j ? T(1) : T(0);
         }
     fro = sum(fro); // also orders the writes above before the reads below
+    int const back = bring_into_range(M, m, red, sum, fro);
     T const eps   = sizeof(T) == 8 ? T(2.220446049250313e-16) : T(1.1920929e-7);
-    T const limit = T(n) * T(n) * eps * eps * fro;
+    T const limit = isinf(fro) ? T(0) : T(n) * T(n) * eps * eps * fro;
     // round-robin pairing (p_i, q_i) of step r: index m-1 fixed in pair 0, the others move by
     // one per step, so a thread keeps the indices of its pairs and advances them; after the
     // m-1 steps of a sweep they are where they began
@@ -422,7 +459,7 @@ __global__ __launch_bounds__(LA_THREADS) void syev_jacobi_kernel(int n, int uppe
                 off += T(2) * v * v;
             }
         off = sum(off);
-        if (off <= limit) {
+        if (__builtin_amdgcn_readfirstlane(int(off <= limit)) != 0) { // the same in every lane
             conv = true;
             break;
         }
@@ -485,7 +522,7 @@ __global__ __launch_bounds__(LA_THREADS) void syev_jacobi_kernel(int n, int uppe
         }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) pos += __shfl_xor(pos, o, 64);
-        if (lane == 0) W[pos] = d;
+        if (lane == 0) W[pos] = ldexp(d, back);
         if (vectors)
             for (int k = lane; k < n; k += 64) A[k + int64_t(pos) * lda] = V[k + int64_t(i) * n];
     }
