@@ -291,6 +291,8 @@ int launch_dense(GemmProblem<T> &P, int blocks_per_cu, hipStream_t stream, size_
     uint64_t slots = P.force_dp == 1 ? tiles : uint64_t(num_cus()) * uint64_t(bpc);
     P.sk           = P.force_dp == 2 ? plan_split_k(tiles, slabs, slots) : plan_stream_k(tiles, slabs, slots);
     P.partial      = nullptr;
+    // a grid of 2^32 threads or more is cut to the remainder without an error
+    if (P.sk.grid >= (uint64_t{1} << 32) / GEMM_THREADS) return fail(EIN_ERROR_UNSUPPORTED, "gemm tile grid too large");
     size_t const piece_bytes = size_t(sk_piece_slots(P.sk)) * BM * BN * sizeof(T);
     if (ws_bytes != nullptr) {
         *ws_bytes = piece_bytes;
