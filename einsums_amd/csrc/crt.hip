@@ -164,7 +164,7 @@ constexpr int CG_SA = CG_TI * 4, CG_SB = CG_TJ * 4;   // 16-byte chunks per oper
 constexpr int CG_DA = CG_SA / 64 / CG_WAVES, CG_DB = CG_SB / 64 / CG_WAVES; // DMA instructions per wave and stage
 
 struct CrtGemm {
-    int64_t m, n, kp;         // rows of a (i), rows of b (j, this panel), padded contraction length
+    int64_t n, kp;            // rows of b (j, this panel), padded contraction length
     int64_t k0, kc;           // contraction steps [k0, k0 + kc) of this launch (multiples of 64)
     int32_t accumulate;       // add to the stored residues instead of overwriting them
     uint32_t items;           // (modulus, tile) pairs
@@ -605,7 +605,6 @@ int gemm_split_crt(GemmProblem<double> P, int nmod, hipStream_t stream) {
     for (int64_t j0 = 0; j0 < P.n; j0 += pn) {
         int64_t const nj = std::min(pn, P.n - j0);
         CrtGemm G{};
-        G.m       = P.m;
         G.n       = nj;
         G.kp      = kp;
         G.a_plane = a_plane;

@@ -38,44 +38,35 @@ constexpr int FOCK_MAX_N = 128;
 template <int MR, int BC>
 __global__ __launch_bounds__(256) void fock_jk_kernel(int n, double const *__restrict__ g, double const *__restrict__ D,
                                                       int64_t ldd, double *__restrict__ J, double *__restrict__ Kp) {
-    constexpr int WAVES = 4, NPL = 1;
+    constexpr int WAVES = 4;
     __shared__ double red[WAVES][BC];
     int const a    = int(blockIdx.x);
     int const ch   = int(blockIdx.y);
     int const wave = int(threadIdx.x) >> 6;
-    int const lane = int(threadIdx.x) & 63;
+    int const lane = int(threadIdx.x) & 63; // d
     int const b0   = ch * BC;
     int const rows = (n - wave + WAVES - 1) / WAVES; // rows c = wave + WAVES*i, i < rows
     int64_t const nn = int64_t(n) * n;
 
-    double x[BC][MR][NPL];
+    double x[BC][MR];
 #pragma unroll
     for (int q = 0; q < BC; ++q) {
         bool const b_in = b0 + q < n;
         double const *__restrict__ slab = g + (int64_t(a) * n + (b_in ? b0 + q : b0)) * nn;
 #pragma unroll
-        for (int i = 0; i < MR; ++i)
-#pragma unroll
-            for (int u = 0; u < NPL; ++u) {
-                int const c = wave + WAVES * i, d = lane + 64 * u;
-                x[q][i][u]  = (b_in && i < rows && d < n) ? slab[int64_t(c) * n + d] : 0.0;
-            }
+        for (int i = 0; i < MR; ++i) {
+            int const c = wave + WAVES * i;
+            x[q][i]     = (b_in && i < rows && lane < n) ? slab[int64_t(c) * n + lane] : 0.0;
+        }
     }
-    double dc[MR][NPL], db[BC][NPL];
+    double dc[MR], db[BC];
 #pragma unroll
-    for (int i = 0; i < MR; ++i)
+    for (int i = 0; i < MR; ++i) {
+        int const c = wave + WAVES * i;
+        dc[i]       = (i < rows && lane < n) ? D[int64_t(c) * ldd + lane] : 0.0;
+    }
 #pragma unroll
-        for (int u = 0; u < NPL; ++u) {
-            int const c = wave + WAVES * i, d = lane + 64 * u;
-            dc[i][u]    = (i < rows && d < n) ? D[int64_t(c) * ldd + d] : 0.0;
-        }
-#pragma unroll
-    for (int q = 0; q < BC; ++q)
-#pragma unroll
-        for (int u = 0; u < NPL; ++u) {
-            int const d = lane + 64 * u;
-            db[q][u]    = (b0 + q < n && d < n) ? D[int64_t(b0 + q) * ldd + d] : 0.0;
-        }
+    for (int q = 0; q < BC; ++q) db[q] = (b0 + q < n && lane < n) ? D[int64_t(b0 + q) * ldd + lane] : 0.0;
 
     double kacc[MR];
 #pragma unroll
@@ -84,12 +75,10 @@ __global__ __launch_bounds__(256) void fock_jk_kernel(int n, double const *__res
     for (int q = 0; q < BC; ++q) {
         double jsum = 0.0;
 #pragma unroll
-        for (int i = 0; i < MR; ++i)
-#pragma unroll
-            for (int u = 0; u < NPL; ++u) {
-                jsum += x[q][i][u] * dc[i][u];
-                kacc[i] += x[q][i][u] * db[q][u];
-            }
+        for (int i = 0; i < MR; ++i) {
+            jsum += x[q][i] * dc[i];
+            kacc[i] += x[q][i] * db[q];
+        }
         // J(a, b): lanes here, the waves after the barrier
         jsum = wave_reduce_sum(jsum);
         if (lane == 0) red[wave][q] = jsum;

@@ -346,8 +346,10 @@ GemmConfig choose_gemm_config(int64_t m, int64_t n, int64_t k, int64_t batch, in
 // Between one round of 64 x 64 tiles and two of 128 x 128 the best choice depends on how the
 // tiles fall on 256 CUs: the fitted choice was 11% (FP64) and 21% (FP32) faster in the mean
 // than a rule on the number of tiles.
-// 96 x 96 is fitted to the products it is for, both operands contiguous along k and aligned
-// (576 x 576 x 9216: 128.2 us in 64 x 64 tiles, 124.0 in 96 x 96).
+// 96 x 96 is fitted to aligned products, both operands contiguous along k (576 x 576 x 9216: 128.2
+// us in 64 x 64 tiles, 124.0 in 96 x 96), and does for unaligned ones: of 24 that the constant of
+// the general fit (1.32) would have put elsewhere, 96 x 96 took 0.96 of the other's time in the
+// mean (0.87 to 1.10, the slower ones with k below 1000).
 namespace {
 struct TileCost {
     int bm, bn, fit; // fit: workgroups resident per CU
