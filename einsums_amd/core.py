@@ -144,7 +144,7 @@ _DESCS_KEPT = 1024
 
 
 def _desc(t: torch.Tensor, idx: str):
-    if not isinstance(idx, str):  # any sequence names labels, but not every one is a key
+    if type(idx) is not str:  # any sequence names labels, but not every one is a key
         if t.dim() != len(idx):
             raise RankError(f"rank of tensor ({t.dim()}) does not match index string {idx!r}")
         return make_desc(idx, t.shape, t.stride())

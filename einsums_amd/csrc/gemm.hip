@@ -349,7 +349,7 @@ GemmConfig choose_gemm_config(int64_t m, int64_t n, int64_t k, int64_t batch, in
 // 96 x 96 is fitted to aligned products, both operands contiguous along k (576 x 576 x 9216: 128.2
 // us in 64 x 64 tiles, 124.0 in 96 x 96), and does for unaligned ones: of 24 that the constant of
 // the general fit (1.32) would have put elsewhere, 96 x 96 took 0.96 of the other's time in the
-// mean (0.87 to 1.10, the slower ones with k below 1000).
+// mean (0.87 to 1.10, the slower ones mostly with k below 1000).
 namespace {
 struct TileCost {
     int bm, bn, fit; // fit: workgroups resident per CU
