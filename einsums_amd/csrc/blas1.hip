@@ -150,6 +150,16 @@ int gemv_impl(char trans, int64_t m, int64_t n, T alpha, T const *A, int64_t lda
     int64_t const leny = notrans ? m : n;
     int64_t const lenx = notrans ? n : m;
     if (leny == 0) return EIN_SUCCESS;
+    // what one grid of fewer than 2^32 threads takes: 64 rows or four columns to a workgroup
+    int64_t const most = int64_t((1 << 24) - 1) * (notrans ? 64 : 4);
+    if (leny > most) {
+        for (int64_t i = 0; i < leny; i += most) {
+            int64_t const c = std::min(most, leny - i);
+            EIN_TRY(gemv_impl<T>(trans, notrans ? c : m, notrans ? n : c, alpha, A + i * (notrans ? 1 : lda), lda, x, incx,
+                                 beta, incy > 0 ? y + i * incy : y - (leny - i - c) * incy, incy, stream));
+        }
+        return EIN_SUCCESS;
+    }
     // negative increments address from the far end, as in BLAS
     if (incx < 0) x = x - (lenx - 1) * incx;
     if (incy < 0) y = y - (leny - 1) * incy;

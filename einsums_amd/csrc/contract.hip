@@ -337,6 +337,7 @@ struct ReduceProblem {
     int32_t parts;  // partials per target written for the finish pass
     int64_t k_chunk;
     T *partial;
+    int64_t first; // wave work of the launch's first wave
 };
 
 // One thread per target point; the K loop walks the digits as an odometer.
@@ -385,7 +386,7 @@ __global__ __launch_bounds__(256) void reduce_wave_kernel(ReduceProblem<T> P) {
     __shared__ T red[4];
     int const lane      = threadIdx.x & 63;
     int const wave      = threadIdx.x >> 6;
-    int64_t const w     = int64_t(blockIdx.x) * 4 + wave;
+    int64_t const w     = P.first + int64_t(blockIdx.x) * 4 + wave;
     int64_t const nwork = P.nt * P.splits;
     // with splits a multiple of 4 the grid holds exactly nwork waves, so only splits == 1
     // (which uses no barrier) returns here
@@ -1140,12 +1141,15 @@ int contract_generic(T c_prefactor, ein_tensor_desc const &C, T *c, T ab_prefact
         EIN_TRY(workspace(stream, size_t(NT) * size_t(R.parts) * sizeof(T), &ws));
         R.partial = static_cast<T *>(ws);
     }
-    int64_t nwaves = NT * R.splits;
-    if (vec)
-        reduce_wave_kernel<T, true><<<uint32_t(ceil_div(nwaves, 4)), 256, 0, stream>>>(R);
-    else
-        reduce_wave_kernel<T, false><<<uint32_t(ceil_div(nwaves, 4)), 256, 0, stream>>>(R);
-    EIN_LAUNCH_CHECK();
+    int64_t const nwaves = NT * R.splits;
+    for (R.first = 0; R.first < nwaves; R.first += WAVE_TILES_MAX) { // a grid holds fewer than 2^32 threads
+        uint32_t const grid = uint32_t(ceil_div(std::min<int64_t>(nwaves - R.first, WAVE_TILES_MAX), 4));
+        if (vec)
+            reduce_wave_kernel<T, true><<<grid, 256, 0, stream>>>(R);
+        else
+            reduce_wave_kernel<T, false><<<grid, 256, 0, stream>>>(R);
+        EIN_LAUNCH_CHECK();
+    }
     if (R.parts > 1) {
         uint32_t grid = uint32_t(std::max<int64_t>(1, std::min<int64_t>(ceil_div(NT, 256), int64_t(cus) * 16)));
         reduce_finish_targets_kernel<T><<<grid, 256, 0, stream>>>(R);
