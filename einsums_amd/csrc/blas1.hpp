@@ -35,6 +35,9 @@ template <typename T>
 int tensor_scale(ein_tensor_desc const &C, T *c, T alpha, hipStream_t stream);
 
 // C = beta*C + alpha*perm(A): C axis i is A axis perm[i] (permute.hip).
+// Estimated microseconds of such a call with alpha == 1 and beta == 0.
+double permute_time_us(int32_t rank, int64_t const *dims_A, int32_t const *perm, int64_t const *strides_A,
+                       int64_t const *strides_C, int elem_bytes);
 template <typename T>
 int permute_tensor(int32_t rank, int64_t const *dims_A, int32_t const *perm, T alpha, T const *A,
                    int64_t const *strides_A, T beta, T *C, int64_t const *strides_C, hipStream_t stream);

@@ -597,31 +597,40 @@ bool folds_to_axis(std::vector<Digit> const &v, int o, int64_t &stride) {
     return stride > 0;
 }
 
-// dst (dense, the listed digits outermost first) = src, src addressed through slot o of
-// each group's digits.
-template <typename T>
-int pack_digits(T const *src, std::vector<std::pair<std::vector<Digit> const *, int>> const &groups, T *dst,
-                hipStream_t stream) {
-    std::vector<int64_t> dims, ss, sd;
-    for (auto const &g : groups)
-        for (auto const &d : *g.first) {
-            dims.push_back(d.e);
-            ss.push_back(d.s[g.second]);
+typedef std::vector<std::pair<std::vector<Digit> const *, int>> DigitGroups; // digits and the slot that addresses them
+
+// The listed digits (outermost first) as axes of a permute between a dense tensor and one
+// addressed through the given slot of each group.
+struct DigitAxes {
+    std::vector<int64_t> dims, dense, strided;
+    std::vector<int32_t> perm;
+    explicit DigitAxes(DigitGroups const &groups) {
+        for (auto const &g : groups)
+            for (auto const &d : *g.first) {
+                dims.push_back(d.e);
+                strided.push_back(d.s[g.second]);
+            }
+        if (dims.empty()) {
+            dims.push_back(1);
+            strided.push_back(1);
         }
-    if (dims.empty()) {
-        dims.push_back(1);
-        ss.push_back(1);
+        dense.resize(dims.size());
+        int64_t pv = 1;
+        for (size_t i = dims.size(); i-- > 0;) {
+            dense[i] = pv;
+            pv *= dims[i];
+        }
+        perm.resize(dims.size());
+        std::iota(perm.begin(), perm.end(), 0);
     }
-    sd.resize(dims.size());
-    int64_t pv = 1;
-    for (size_t i = dims.size(); i-- > 0;) {
-        sd[i] = pv;
-        pv *= dims[i];
-    }
-    std::vector<int32_t> perm(dims.size());
-    std::iota(perm.begin(), perm.end(), 0);
-    return permute_tensor<T>(int32_t(dims.size()), dims.data(), perm.data(), T(1), src, ss.data(), T(0), dst, sd.data(),
-                             stream);
+};
+
+// dst (dense, the listed digits outermost first) = src.
+template <typename T>
+int pack_digits(T const *src, DigitGroups const &groups, T *dst, hipStream_t stream) {
+    DigitAxes const x(groups);
+    return permute_tensor<T>(int32_t(x.dims.size()), x.dims.data(), x.perm.data(), T(1), src, x.strided.data(), T(0), dst,
+                             x.dense.data(), stream);
 }
 
 // Transpose-transpose-GEMM: an operand whose digits do not fold into one strided matrix is
@@ -631,13 +640,14 @@ int pack_digits(T const *src, std::vector<std::pair<std::vector<Digit> const *, 
 // into C by the permute. Digit orders are chosen to fold as much as possible. The route
 // is taken (`taken` = true) when nothing is packed, or when packing, dense product and staging
 // are put below gather_us, the estimate of the gather GEMM (0: only if nothing is packed).
-// FP64 is fitted to "mbej <- jnfb, mnef" (o 9..32, v 43..104) and "pqrs <- pmrs, mq" (36..100): over
-// 22 of them the choice loses at most 6% against the better route, where 0.45 of the dense
-// product's time as the line for the extra traffic took the gather for 17 x 51 (FP64 145 us, packed
-// 66), 13 x 77 (207, 92), 20 x 60 (133, 105), 16 x 64 (82, 71). FP32 is fitted to 290 products, those
-// two and six forms of "acdb <- aebf, fced" with extents 6..56, timed by both routes: it loses 0.06%
-// in the mean and at most 8% (mbej 24, 96: packed 262 us, gathered 320; "pqrs" 64: 99 and 64), and
-// chooses the same up to 1.5 and 1.9. FP64 on 286 products of those kinds: 0.2%, at most 14%.
+// The factors are fitted to "mbej <- jnfb, mnef" (o 9..32, v 24..110), "pqrs <- pmrs, mq" (32..100) and
+// six forms of "acdb <- aebf, fced" with extents 6..56, timed by both routes: over 374 of them in each
+// type FP32 loses 0.3% in the mean against the better route and at most 7% (mbej 24, 96: packed 262
+// us, gathered 320; "pqrs" 64: 99 and 64), FP64 1.5%, most of it where the wave kernel takes a small
+// one. What packing takes is priced by its permutes: with one rate for all of them, products were
+// packed whose inner extents are too short for it ("cadb <- eafb, fdec" 8,2,5,187,276,88 FP64 285 us,
+// gathered 199; "abcd <- aecf, ebfd" 3,145,13,129,76,12 FP32 140 and 80). A line at 0.45 of the dense
+// product's time took the gather for mbej 17 x 51 (FP64 145 us, packed 66), 13 x 77 (207, 92).
 constexpr double GATHER_SLOWER[] = {1.65, 1.3}, GATHER_UNALIGNED[] = {1.5, 1.3}; // FP64, FP32
 
 template <typename T>
@@ -678,7 +688,9 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
                            (ch.c_ok ? 0.0 : double(NB) * M * N);
                 if (best.moved < 0.0 || ch.moved < best.moved) best = ch;
             }
-    int const launches   = int(!best.a_ok) + int(!best.b_ok) + int(!best.c_ok);
+    int const launches = int(!best.a_ok) + int(!best.b_ok) + int(!best.c_ok);
+    DigitGroups const a_groups{{&best.bt, 0}, {&best.m, 0}, {&best.k, 0}}, b_groups{{&best.bt, 1}, {&best.n, 0}, {&best.k, 1}},
+        x_groups{{&best.bt, 2}, {&best.n, 1}, {&best.m, 1}};
     if (!forced && launches > 0) {
         bool below;
         if (sizeof(T) == 8 && gemm_split_on()) {
@@ -687,13 +699,21 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
             double const t_extra = 2.0 * sizeof(T) * best.moved / 4e12 + 5e-6 * launches;
             below                = t_extra < 0.45 * t_gemm;
         } else {
+            if (gather_us == 0.0) return EIN_SUCCESS;
             auto unaligned = [&](bool ok, int64_t const *s, int64_t rows, T const *ptr) {
                 return !(ok ? choose_staging<T>(128, s[1], s[2], s[0], NB, rows, K, ptr).wide : K * int64_t(sizeof(T)) % 16 == 0);
             };
             int const ua = unaligned(best.a_ok, best.as, M, a), ub = unaligned(best.b_ok, best.bs, N, b);
             double const dense = gemm_time_us(M, N, K, NB, int(sizeof(T)), true, ua + ub);
-            double const extra = 2e6 * sizeof(T) * best.moved / 5e12 + (sizeof(T) == 8 ? 4.0 : 3.0) * launches;
-            below              = dense + extra < 0.95 * gather_us;
+            auto move          = [](DigitGroups const &groups, bool to_dense) {
+                DigitAxes const x(groups);
+                return permute_time_us(int32_t(x.dims.size()), x.dims.data(), x.perm.data(),
+                                                (to_dense ? x.strided : x.dense).data(), (to_dense ? x.dense : x.strided).data(),
+                                                int(sizeof(T)));
+            };
+            double const extra = (best.a_ok ? 0.0 : move(a_groups, true)) + (best.b_ok ? 0.0 : move(b_groups, true)) +
+                                 (best.c_ok ? 0.0 : move(x_groups, false));
+            below = dense + extra < 0.95 * gather_us;
         }
         if (!below) return EIN_SUCCESS;
     }
@@ -727,7 +747,7 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
         P.a_sk = best.as[2];
     } else {
         T *pa = reinterpret_cast<T *>(ws);
-        EIN_TRY(pack_digits<T>(a, {{&best.bt, 0}, {&best.m, 0}, {&best.k, 0}}, pa, stream));
+        EIN_TRY(pack_digits<T>(a, a_groups, pa, stream));
         P.A    = pa;
         P.a_sb = M * K;
         P.a_sm = K;
@@ -740,7 +760,7 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
         P.b_sk = best.bs[2];
     } else {
         T *pb = reinterpret_cast<T *>(ws + a_bytes);
-        EIN_TRY(pack_digits<T>(b, {{&best.bt, 1}, {&best.n, 0}, {&best.k, 1}}, pb, stream));
+        EIN_TRY(pack_digits<T>(b, b_groups, pb, stream));
         P.B    = pb;
         P.b_sb = N * K;
         P.b_sn = K;
@@ -763,23 +783,9 @@ int contract_ttgt(std::vector<Digit> const &vb, std::vector<Digit> const &vm, st
     EIN_TRY(gemm_dispatch<T>(P, stream));
     if (!best.c_ok) {
         // C = beta*C + X over the (batch, N, M) digits
-        std::vector<int64_t> dims, sx, sc;
-        int64_t pv = 1;
-        std::vector<std::pair<std::vector<Digit> const *, int>> const order = {{&best.bt, 2}, {&best.n, 1}, {&best.m, 1}};
-        for (auto const &g : order)
-            for (auto const &d : *g.first) {
-                dims.push_back(d.e);
-                sc.push_back(d.s[g.second]);
-            }
-        sx.resize(dims.size());
-        for (size_t i = dims.size(); i-- > 0;) {
-            sx[i] = pv;
-            pv *= dims[i];
-        }
-        std::vector<int32_t> perm(dims.size());
-        std::iota(perm.begin(), perm.end(), 0);
-        EIN_TRY(permute_tensor<T>(int32_t(dims.size()), dims.data(), perm.data(), T(1), X, sx.data(), beta, c, sc.data(),
-                                  stream));
+        DigitAxes const x(x_groups);
+        EIN_TRY(permute_tensor<T>(int32_t(x.dims.size()), x.dims.data(), x.perm.data(), T(1), X, x.dense.data(), beta, c,
+                                  x.strided.data(), stream));
     }
     return EIN_SUCCESS;
 }
