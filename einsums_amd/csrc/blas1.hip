@@ -425,13 +425,13 @@ int dot_noalloc_f64(int64_t n, double alpha, double const *x, int64_t incx, doub
 // A(i,j) = beta*A(i,j) + alpha*x(i)*y(j) over rows of stride rs and columns of stride lda.
 // HBM-bound: A is written once, and read once unless beta == 0. A workgroup is 2^tr threads
 // along the rows times 256 / 2^tr along the columns; a thread owns VEC consecutive rows (one
-// 16-byte access) of GER_COLS columns, whose reads are issued together. The row width follows
+// 16-byte access) of COLS columns, whose reads are issued together. The row width follows
 // m, so that a short m leaves no lane idle: the rank-0 times tensor product of a gradient is
 // a 1 x N outer product, which a fixed 64-row block ran with one lane in 64 (16.8M doubles
 // 1706 us plus 21 us to zero them first; in this form, with the factor on A fused, 46 us = 5.8 TB/s).
 constexpr int GER_COLS = 4;
 
-template <typename T, int VEC>
+template <typename T, int VEC, int COLS>
 __global__ __launch_bounds__(256) void ger_kernel(int64_t m, int64_t n, T alpha, T const *__restrict__ x, int64_t incx,
                                                   T const *__restrict__ y, int64_t incy, T beta, T *__restrict__ A,
                                                   int64_t rs, int64_t lda, int tr) {
@@ -445,18 +445,18 @@ __global__ __launch_bounds__(256) void ger_kernel(int64_t m, int64_t n, T alpha,
     T xi[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) xi[v] = alpha * x[(i + v) * incx];
-    int64_t const step = int64_t(cols) * GER_COLS;
+    int64_t const step = int64_t(cols) * COLS;
     for (int64_t j0 = int64_t(blockIdx.y) * step + lc; j0 < n; j0 += int64_t(gridDim.y) * step) {
-        Vec c[GER_COLS];
-        T yj[GER_COLS];
+        Vec c[COLS];
+        T yj[COLS];
 #pragma unroll
-        for (int u = 0; u < GER_COLS; ++u) {
+        for (int u = 0; u < COLS; ++u) {
             int64_t const j = j0 + u * cols;
             yj[u]           = j < n ? y[j * incy] : T(0);
             if (beta != T(0) && j < n) c[u] = *reinterpret_cast<Vec const *>(A + i * rs + j * lda);
         }
 #pragma unroll
-        for (int u = 0; u < GER_COLS; ++u) {
+        for (int u = 0; u < COLS; ++u) {
             int64_t const j = j0 + u * cols;
             if (j >= n) break;
 #pragma unroll
@@ -493,16 +493,20 @@ int ger_impl(int64_t m, int64_t n, T alpha, T const *x, int64_t incx, T const *y
     int64_t const r  = vec ? m / VW : m; // threads along the rows
     int tr           = 0;
     while (tr < 8 && (int64_t{1} << tr) < r) ++tr;
-    int64_t const cb = std::min<int64_t>(ceil_div(n, int64_t(256 >> tr) * GER_COLS), 65535);
+    // one column a thread for few columns of a small A: the call is one round of latencies, which
+    // four columns make longer (FP64 with a factor on A 38 x 1449 2.6 -> 2.2 us, 64 x 4096 2.6 -> 2.3),
+    // but 300 x 300 2.1, so 2.3, and 500 x 1000 FP32 2.4 and 2.7
+    int64_t const per_block = 256 >> tr;
+    bool const one          = n <= 64 && m <= (1 << 18) / n;
+    int64_t const cb        = std::min<int64_t>(ceil_div(n, per_block * (one ? 1 : GER_COLS)), 65535);
     // rows of one launch: a grid holds fewer than 2^32 threads (and is cut without an error beyond)
     int64_t const rows = int64_t((1 << 24) - 1) * (int64_t{1} << tr) * (vec ? VW : 1);
+    auto const kernel  = vec ? (one ? ger_kernel<T, VW, 1> : ger_kernel<T, VW, GER_COLS>)
+                             : (one ? ger_kernel<T, 1, 1> : ger_kernel<T, 1, GER_COLS>);
     for (int64_t i0 = 0; i0 < m; i0 += rows) {
         int64_t const mi = std::min(rows, m - i0);
         dim3 const grid{uint32_t(ceil_div(vec ? mi / VW : mi, int64_t{1} << tr)), uint32_t(cb)};
-        if (vec)
-            ger_kernel<T, VW><<<grid, 256, 0, stream>>>(mi, n, alpha, x + i0 * incx, incx, y, incy, beta, A + i0 * rs, rs, lda, tr);
-        else
-            ger_kernel<T, 1><<<grid, 256, 0, stream>>>(mi, n, alpha, x + i0 * incx, incx, y, incy, beta, A + i0 * rs, rs, lda, tr);
+        kernel<<<grid, 256, 0, stream>>>(mi, n, alpha, x + i0 * incx, incx, y, incy, beta, A + i0 * rs, rs, lda, tr);
         EIN_LAUNCH_CHECK();
     }
     return EIN_SUCCESS;
