@@ -690,15 +690,28 @@ int gemm_strided_impl(GemmProblem<T> P, GemmConfig const *force, hipStream_t str
         return !sa.krow || sa.wide;
     };
     if (force && cfg.bm == 256 && !rows_256()) cfg.bm = 128;
-    if (sizeof(T) == 4 && !force && cfg.bm == 128 && cfg.bn == 128 && rows_256() &&
-        ceil_div(P.m, 256) * ceil_div(P.n, 128) * P.batch >= 2 * int64_t(num_cus())) {
+    if (sizeof(T) == 4 && !force && cfg.bm == 128 && cfg.bn == 128 && rows_256() && P.k >= 256 &&
+        2 * ceil_div(P.m, 256) == ceil_div(P.m, 128)) {
         // FP32 slabs of 128 x 128 are half as long in time as FP64's, and what they stage per
-        // MFMA is what holds them back (without the staging 140 TFLOP/s, with it 119): from two
-        // rounds of 256 x 128 tiles on, a wave of 128 x 64 stages a quarter less. 4096^3 NN
-        // 1155 -> 1066 us, NT 1128 -> 1077, TN 1060 -> 1037; with fewer tiles the last round costs
-        // more than that (3000^3, 288 tiles: TN 453 -> 474; 1536^3, 72 tiles: NN 81 -> 88).
-        cfg.bm            = 256;
-        cfg.blocks_per_cu = 0;
+        // MFMA is what holds them back (without the staging 140 TFLOP/s, with it 119): a wave of
+        // 128 x 64 stages a quarter less, but a tile costs more to begin and to end, and twice to
+        // cut. So no row of tiles may be half empty (384 x 384 x 400, 200 products: 297 us with
+        // 256 rows, 221 with 128), k must be long (4096 x 4096 x 16 20.2 us and 18.1, x 48 27.6 and 26.2,
+        // x 400 114.8 and 122.2), and the rounds whole from two on (3200 x 5120 x 400, 520 tiles: 128 and 122), or,
+        // with A k-major and B contiguous along k, at least three and k from 512 (11712 x 3392 x 1424 943
+        // and 987; both contiguous along k 0.93 to 1.02 of the time with 128 rows, both k-major 1.01 to
+        // 1.14). 4096^3 NN 1155 -> 1066 us, NT 1128 -> 1077, TN 1060 -> 1037. Over 467 products of 512
+        // such tiles and more the rule gains 0.3% in the mean and loses at most 1.2%; the tile wherever
+        // there are two rounds of it lost 15%.
+        int64_t const tiles256  = ceil_div(P.m, 256) * ceil_div(P.n, 128) * P.batch, cus = num_cus();
+        OperandStaging const sa = choose_staging<T>(256, P.a_sm, P.a_sk, P.a_sb, P.batch, P.m, P.k, P.A);
+        OperandStaging const sb = choose_staging<T>(128, P.b_sn, P.b_sk, P.b_sb, P.batch, P.n, P.k, P.B);
+        double const rounds     = double(tiles256) / double(cus);
+        bool const whole        = !sa.krow && !sb.krow ? tiles256 % cus == 0 : rounds >= 0.97 * std::ceil(rounds);
+        if (tiles256 >= 2 * cus && (whole || (!sa.krow && sb.krow && tiles256 >= 3 * cus && P.k >= 512))) {
+            cfg.bm            = 256;
+            cfg.blocks_per_cu = 1;
+        }
     }
     if (!force) {
         OperandStaging const sa = choose_staging<T>(128, P.a_sm, P.a_sk, P.a_sb, P.batch, P.m, P.k, P.A);
