@@ -95,7 +95,7 @@ __device__ __forceinline__ int bring_into_range(T *M, int m, T *red, Sum const &
     constexpr T LEAST = sizeof(T) == 8 ? T(1e-200) : T(1e-20), MOST = sizeof(T) == 8 ? T(1e300) : T(1e37);
     // the same in every lane; the compiler has to know, or the sweeps' scalar state goes to vectors
     auto uniform = [](bool x) { return __builtin_amdgcn_readfirstlane(int(x)) != 0; };
-    if (uniform(fro >= LEAST && fro <= MOST)) return 0;
+    if (__builtin_expect(uniform(fro >= LEAST && fro <= MOST), 1)) return 0;
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     T big = T(0);
     for (int x = threadIdx.x; x < m * (m + 1) / 2; x += blockDim.x) big = fmax(big, fabs(M[x]));
